@@ -28,7 +28,8 @@ struct AttnArgs {
   int H, KVH;
   float eps, scale;
   float* out;    // [n_tok][H*128]
-  Q8Mut out_q8;  // Q8 blocks of out
+  Q8Mut out_q8;      // decode: Q8 blocks of out
+  Q8Tiles out_tiles; // prefill: the same in 32-token tiles
   uint32_t* err; // device error word (nullable): an expired bounded wait sets kErrAttnExp
   // test knob of the decode softmax's exact parallel sum (0 in use): shifts
   // the walk's predicted binades so that runs replay (block_softmax_sum)

@@ -1510,10 +1510,7 @@ __global__ void __launch_bounds__(512) k_attn_pv_pre(AttnArgs a) {
       const uint32_t tok = tok0 + (uint32_t)(cb / G);
       const uint32_t col = (uint32_t)(g * G + cb % G) * kHd + d;
       ((RLH_GLOBAL float*)a.out)[(size_t)tok * qd + col] = o[i];
-      const uint32_t nbq = (uint32_t)qd / 32;
-      Q8Out ot{a.out_q8.qs + (size_t)tok * qd, a.out_q8.d + (size_t)tok * nbq, a.out_q8.s + (size_t)tok * nbq,
-               a.out_q8.s16 + (size_t)tok * nbq * 2};
-      q8_quant_block32(o[i], ot, col / 32);
+      q8_quant_block32(o[i], a.out_tiles, tok, col / 32);
     }
   }
 }

@@ -268,6 +268,7 @@ int ensure_device() {
   static bool lds_set = false;
   if (!lds_set) {
     if (!mv_set_max_lds(150 * 1024)) return fail(RLH_EDEVICE, "matvec LDS attribute");
+    if (!gemm_set_max_lds()) return fail(RLH_EDEVICE, "prefill product LDS attribute");
     lds_set = true;
   }
   return RLH_OK;
@@ -328,7 +329,7 @@ struct rlh_cache {
   uint32_t bcap = 0;
   float *xb = nullptr, *qb = nullptr, *kb = nullptr, *vb = nullptr, *attnb = nullptr, *gb = nullptr, *ub = nullptr,
         *scoresb = nullptr, *xnb = nullptr;  // xnb: f32 rmsnorm rows (inputs of f32-route products)
-  Q8Buf act_eb{}, act_qb{}, act_fb{};
+  Q8Tiles act_eb{}, act_qb{}, act_fb{};
   uint32_t* tokb = nullptr;   // token ids of the whole call
   uint32_t* posb = nullptr;   // first position of every chunk
   uint64_t tokb_cap = 0, posb_cap = 0;
@@ -805,9 +806,8 @@ static void cache_free(rlh_cache* c) {
                   c->pi, c->dbg};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
-  void* bptrs[] = {c->xb, c->qb, c->kb, c->vb, c->attnb, c->gb, c->ub, c->scoresb, c->xnb, c->act_eb.qs, c->act_eb.d,
-                   c->act_eb.s, c->act_eb.s16, c->act_qb.qs, c->act_qb.d, c->act_qb.s, c->act_qb.s16, c->act_fb.qs,
-                   c->act_fb.d, c->act_fb.s, c->act_fb.s16, c->tokb, c->posb};
+  void* bptrs[] = {c->xb, c->qb, c->kb, c->vb, c->attnb, c->gb, c->ub, c->scoresb, c->xnb, c->act_eb.p, c->act_qb.p,
+                   c->act_fb.p, c->tokb, c->posb};
   for (void* p : bptrs)
     if (p) (void)hipFree(p);
   if (c->host_st) (void)hipHostFree(c->host_st);
@@ -825,6 +825,12 @@ static int alloc_q8(Q8Buf& b, uint64_t n) {
   if (hipMalloc((void**)&b.qs, n) != hipSuccess || hipMalloc((void**)&b.d, n / 32 * 4) != hipSuccess ||
       hipMalloc((void**)&b.s, n / 32 * 4) != hipSuccess || hipMalloc((void**)&b.s16, n / 16 * 4) != hipSuccess)
     return fail(RLH_ENOMEM, "hipMalloc Q8 activation");
+  return RLH_OK;
+}
+
+static int alloc_q8_tiles(Q8Tiles& b, uint64_t n, uint64_t cols) {
+  if (hipMalloc((void**)&b.p, q8_tiles_bytes(n, cols)) != hipSuccess) return fail(RLH_ENOMEM, "hipMalloc Q8 tiles");
+  b.nsb = (uint32_t)(cols / 256);
   return RLH_OK;
 }
 
@@ -973,9 +979,9 @@ static int ensure_batch(rlh_cache* c) {
             hipMalloc((void**)&c->ub, B * F * 4) == hipSuccess && hipMalloc((void**)&c->xnb, B * E * 4) == hipSuccess &&
             hipMalloc((void**)&c->scoresb, (size_t)B * cfg.n_head * c->max_ctx * 4) == hipSuccess;
   if (!ok) return fail(RLH_ENOMEM, "prefill workspace allocation failed");
-  int rc = alloc_q8(c->act_eb, B * E);
-  if (!rc) rc = alloc_q8(c->act_qb, B * qd);
-  if (!rc) rc = alloc_q8(c->act_fb, B * F);
+  int rc = alloc_q8_tiles(c->act_eb, B, E);
+  if (!rc) rc = alloc_q8_tiles(c->act_qb, B, qd);
+  if (!rc) rc = alloc_q8_tiles(c->act_fb, B, F);
   if (rc) return rc;
   c->bcap = B;
   return RLH_OK;
@@ -1026,14 +1032,14 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
     // products give the last n % 4 tokens of the call the single-token order)
     const uint64_t n4_all = n - n % 4;
     const uint32_t n4 = (uint32_t)std::min<uint64_t>(mtok, n4_all > c0 ? n4_all - c0 : 0);
-    auto product_on = [&](hipStream_t s, const DevMat& w, const Q8Buf& q8, const float* xf, float* y,
+    auto product_on = [&](hipStream_t s, const DevMat& w, const Q8Tiles& q8, const float* xf, float* y,
                           float* resid) {
       if (gemm_supported(w.ty))
         launch_gemm(s, w, q8, mtok, y, resid);
       else
         launch_gemm_f32(s, w, xf, mtok, n4, y, resid);
     };
-    auto product = [&](const DevMat& w, const Q8Buf& q8, const float* xf, float* y, float* resid) {
+    auto product = [&](const DevMat& w, const Q8Tiles& q8, const float* xf, float* y, float* resid) {
       product_on(st, w, q8, xf, y, resid);
     };
     float* xn = m->f32_route ? c->xnb : nullptr;  // f32 rmsnorm rows, when a product needs them
@@ -1105,7 +1111,7 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
       a.eps = eps;
       a.scale = scale;
       a.out = c->attnb;
-      a.out_q8 = c->act_qb;
+      a.out_tiles = c->act_qb;
       a.err = err_word(c);
       launch_attn_scores(st, a, false);
       launch_attn_softmax(st, a);
@@ -1121,7 +1127,7 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
       }
       // h over the gate rows in place when ffn_down takes the f32 route
       const bool hf = !gemm_supported(L.down.ty);
-      launch_swiglu_q8(st, c->gb, c->ub, mtok * cfg.n_ff, c->act_fb, hf ? c->gb : nullptr);
+      launch_swiglu_q8(st, c->gb, c->ub, mtok, c->act_fb, hf ? c->gb : nullptr);
       product(L.down.dm, c->act_fb, c->gb, nullptr, c->xb);
       if (c->debug && c->dbg && c0 < c->dbg_tokens) {
         const uint64_t nd = std::min<uint64_t>(mtok, c->dbg_tokens - c0);
@@ -1370,19 +1376,17 @@ int rlh_matmul_batch(uint32_t ty, const void* w, uint64_t rows, uint64_t cols, c
   if (rc) return rc;
   hipStream_t st = op_stream();
   const uint64_t nv = n * cols;
-  DevBuf<float> dx, dy, dd;
-  DevBuf<int8_t> dq;
-  DevBuf<int32_t> ds, ds16;
-  if (dx.alloc(nv) || dy.alloc(n * rows) || dq.alloc(nv) || dd.alloc(nv / 32) || ds.alloc(nv / 32) ||
-      ds16.alloc(nv / 16)) {
+  DevBuf<float> dx, dy;
+  DevBuf<uint8_t> dq;
+  if (dx.alloc(nv) || dy.alloc(n * rows) || dq.alloc(q8_tiles_bytes(n, cols))) {
     free_tensor(t);
     return fail(RLH_ENOMEM, "hipMalloc");
   }
   // quantize_q8 of every token row (ops.rs:207-209), then the products
-  const Q8Buf act{dq.p, dd.p, ds.p, ds16.p};
+  const Q8Tiles act{dq.p, (uint32_t)(cols / 256)};
   hipError_t e = hipMemcpyAsync(dx.p, xs, nv * 4, hipMemcpyHostToDevice, st);
   if (gemm_supported(ty)) {
-    launch_quantize_q8(st, dx.p, (uint32_t)nv, act);
+    launch_quantize_q8(st, dx.p, (uint32_t)n, act);
     launch_gemm(st, t.dm, act, (uint32_t)n, dy.p, nullptr);
   } else {  // the f32 route (ops.rs:237-312): no activation quantization
     launch_gemm_f32(st, t.dm, dx.p, (uint32_t)n, (uint32_t)(n - n % 4), dy.p, nullptr);

@@ -5,25 +5,22 @@
 // Exactness: for every (token, row) the output is the reference's f32 chain
 // `total += term` over the row's terms in index order; each term is formed
 // with the reference's expression (simd.rs:581 Q4_K, 663 Q6_K, 863 Q4_0,
-// 891 Q8_0). The integer block dots inside the terms come from
-// v_mfma_i32_16x16x32_i8 and are exact:
-//   Q4_K  unsigned nibbles (0..15) x Q8 bytes, one MFMA per 32-value block;
-//   Q6_K  q = u - 32 as signed bytes, so the MFMA gives sum(q a) = ss - 32 sa
-//         exactly, which is what (ss as f32 - 32.0 * sa as f32) evaluates to
-//         (both are integers below 2^24); one MFMA per 16-value half, the
-//         other half of the operand zeroed;
-//   Q8_0  signed bytes; Q4_0 nibble - 8, i.e. i0 + i1 - 8 * sum exactly.
-// The per-element float epilogue runs on the VALU and dominates the cost.
-//
-// Tiling: a block owns 64 tokens x 64 rows; 4 waves of 32 x 32, each 2 x 2
-// MFMA tiles of 16 x 16. Per super-block (256 values) the block stages the
-// 64 tokens' Q8 bytes and block scales into LDS (double buffered, copied
-// through registers); every lane loads the weight bytes of its row straight
-// from the tiled layout, one super-block ahead. Block b runs on XCD b % 8; the blocks
-// of one XCD walk the token tiles of a row tile first, so each weight tile
-// is fetched into that XCD's L2 once and reused by all token tiles.
+// 891 Q8_0). The integer block dots inside the terms come from int8 MFMA and
+// are exact. Three identities keep work off the VALU, whose f32 combine is
+// what bounds these kernels; none of them changes a rounding:
+//   * the MFMA starts from kBase, the bits of an f32 in the middle of its
+//     binade, so its i32 result read as f32 is that f32 + dot * 2^-26
+//     (|dot| < 2^21), and one f32 subtraction gives dot * 2^-26 exactly; the
+//     power of two goes into the row's scale. A v_sub_f32 issues every 2.3
+//     cycles per SIMD (two waves or more ready), a v_cvt_f32_i32 every 4.1;
+//   * Q6_K and Q4_0 weights enter the MFMA as 4 q and 16 q (the bit field
+//     moved to the top of its byte, the sign bit flipped), and their scale is
+//     a quarter or a sixteenth: powers of two, exact on both sides;
+//   * Q4_K's dmin*m * sum products are a rank-1 product, one f32 MFMA of
+//     depth 1 from C = 0 (each result is the product rounded once).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
 
 #include "gemm.h"
 #include "rlh_device.h"
@@ -33,663 +30,513 @@ namespace rlh {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x32_t __attribute__((ext_vector_type(32)));
 typedef RLH_LDS uint8_t lbyte;
 
-constexpr uint32_t kTile = 64;                          // tokens and rows per block
-constexpr uint32_t kXStride = 272;                      // LDS bytes per token per super-block (16-byte pad)
-constexpr uint32_t kXBytes = kTile * kXStride;          // 17408
-constexpr uint32_t kDBytes = kTile * 8 * 4;             // da of 8 blocks per token, block-major [8][64]
-constexpr uint32_t kRBytes = kTile * 4 * 16;            // Q4_K row scales: [4 groups][64 rows] float4
-constexpr uint32_t kStageBytes = kXBytes + 2 * kDBytes + kRBytes;  // + sums as f32 (Q4_K), + row scales
+// The MFMA's C operand: an inline constant of the instruction set, 1 / (2 pi)
+// as f32, taken as an integer; kBaseF is its value and 2^-26 its unit.
+constexpr int kBase = 0x3e22f983;
+constexpr float kBaseF = 0x1.45f306p-3f, kUnit = 67108864.0f;  // 2^26
 
-__device__ __forceinline__ uint64_t g8(const uint8_t* p) { return *(const RLH_GLOBAL uint64_t*)p; }
-__device__ __forceinline__ u32x4_t g16(const uint8_t* p) { return *(const RLH_GLOBAL u32x4_t*)p; }
-__device__ __forceinline__ long l8(const lbyte* p) { return *(const RLH_LDS long*)p; }
-
-__device__ __forceinline__ v4i mfma(long a, uint64_t b) {
-  const v4i z = {0, 0, 0, 0};
-  return __builtin_amdgcn_mfma_i32_16x16x32_i8(a, (long)b, z, 0, 0, 0);
-}
-
-// Bytes of item (row, j) in the tiled layout: byte o < 16 * (ib / 16) lies
-// at base + (o / 16) * 1024 + o % 16; the ib % 16 tail bytes at `tail`.
-struct ItemPtr {
-  const uint8_t* base;
-  const uint8_t* tail;
+// Shape of a block. Four waves, 2 token waves x 2 row waves; a wave computes
+// a tile of MT tokens x MT rows (MT = the MFMA's edge), tokens in the result
+// registers, rows across the lanes.
+//   MT 32: 64 tokens x 64 rows per block, stages of half a super-block (128
+//          values of the columns), two of them;
+//   MT 16: 32 tokens x 32 rows per block, four stages of a super-block (few
+//          blocks per CU: the copies run further ahead).
+// A stage is copied into LDS by DMA, half by half: the activation tiles'
+// quants, scales and sums as they lie in memory (Q8Tiles), the weight rows'
+// 16-byte chunks as [chunk][row], and Q6_K's f16 d in its 4-byte word. Half
+// super-blocks and at most 128 registers because four MT 32 blocks then fit
+// a CU: a SIMD issues f32 adds and multiplies of two waves side by side (2.3
+// cycles each, 4.6 when one wave is ready), and with four waves per SIMD two
+// are ready most of the time (Q8_0, 24576 x 4096 x 512 tokens: 234 us with
+// whole super-blocks and two blocks per CU, 194 with four).
+template <uint32_t TY, int MT>
+struct Geo {
+  static constexpr bool kSums = TY == RLH_TYPE_Q4_K;
+  static constexpr uint32_t kActTiles = MT == 32 ? 2 : 1;
+  static constexpr uint32_t kTok = 32 * kActTiles;
+  static constexpr uint32_t kRows = 2 * MT;
+  static constexpr uint32_t kHalves = MT == 32 ? 1 : 2;  // halves of a super-block per stage
+  static constexpr uint32_t kStages = MT == 32 ? 2 : 4;
+  static constexpr uint32_t kCh = TY == RLH_TYPE_Q8_0 ? 9 : TY == RLH_TYPE_Q6_K ? 7 : 5;  // chunks of a half
+  static constexpr uint32_t kActI = 4 * kActTiles + (MT == 32 && kSums ? 2 : 1);          // 1 KB copies
+  static constexpr uint32_t kWI = (kCh * kRows * 16 + 1023) / 1024;
+  static constexpr uint32_t kTailI = TY == RLH_TYPE_Q6_K ? 1 : 0;  // a 256-byte copy
+  static constexpr uint32_t kCopies = kActI + kWI + kTailI;
+  static constexpr uint32_t kPerWave = (kCopies + 3) / 4;  // copies of a half per wave
+  static constexpr uint32_t kDOff = kActTiles * 4096;      // scales, then sums: 512 bytes per tile
+  static constexpr uint32_t kWOff = kActI * 1024, kTailOff = kWOff + kWI * 1024;
+  static constexpr uint32_t kHalfBytes = kTailOff + kTailI * 256;
+  static constexpr uint32_t kStageBytes = kHalves * kHalfBytes;
+  static constexpr uint32_t kLds = kStages * kStageBytes;
+  // chunk of the item that staged chunk c of half h holds
+  __device__ __forceinline__ static uint32_t chunk(uint32_t c, uint32_t h) {
+    if (TY == RLH_TYPE_Q4_K) return c ? c + 4 * h : 0;
+    if (TY == RLH_TYPE_Q6_K) return c < 4 ? c + 4 * h : c < 6 ? c + 4 + 2 * h : 12;
+    if (TY == RLH_TYPE_Q8_0) return c < 8 ? c + 8 * h : 16;
+    return c < 4 ? c + 4 * h : 8;
+  }
 };
-__device__ __forceinline__ ItemPtr item_ptr(const DevMat& w, uint32_t row, uint32_t j) {
-  const uint32_t rt = row / w.tr, jt = j / w.tj, l = (j % w.tj) * w.tr + row % w.tr;
-  const uint8_t* tb = w.a + ((size_t)rt * w.ntj + jt) * 64 * w.ib;
-  const uint32_t ch = w.ib / 16;
-  return ItemPtr{tb + l * 16, tb + ch * 1024 + l * (w.ib - ch * 16)};
-}
-__device__ __forceinline__ const uint8_t* at(const ItemPtr& p, uint32_t o) { return p.base + (o >> 4) * 1024 + (o & 15); }
 
-// Lane coordinates inside the block: lane = 16 q + i16; wave = 2 rw + tw.
-struct Lane {
-  uint32_t q, i16, tw, rw;
-};
-
-// View of a staged super-block. The token scales and sums are block-major
-// ([block][token], so the four tokens a lane owns are one 16-byte read) for
-// Q4_K, Q8_0 and Q4_0, token-major ([token][block]) for Q6_K.
-struct StageView {
-  const lbyte* xs;            // [64][kXStride] Q8 bytes
-  const RLH_LDS float* d;     // block scales
-  const RLH_LDS float* s;     // Q4_K: block sums, as f32 (exact: |sum| <= 4064), block-major
-  const RLH_LDS f32x4_t* rs;  // Q4_K, [4][64]: {d*sc, dmin*m} of sub-blocks 2g, 2g+1 of each row
-};
-
-__device__ __forceinline__ StageView view(const lbyte* buf) {
-  return StageView{buf, (const RLH_LDS float*)(buf + kXBytes), (const RLH_LDS float*)(buf + kXBytes + kDBytes),
-                   (const RLH_LDS f32x4_t*)(buf + kXBytes + 2 * kDBytes)};
-}
-
-// The lane's four tokens' values of block kb (scales or sums).
-__device__ __forceinline__ f32x4_t tok4(const RLH_LDS float* t, const Lane& ln, uint32_t tr, uint32_t kb) {
-  return *(const RLH_LDS f32x4_t*)(t + kb * kTile + 32 * ln.tw + 16 * tr + 4 * ln.q);
-}
-
-// A operands of block kb (0..7 inside the super-block) for token tile tr.
-__device__ __forceinline__ long a_frag(const StageView& v, const Lane& ln, uint32_t tr, uint32_t kb) {
-  const uint32_t tok = 32 * ln.tw + 16 * tr + ln.i16;
-  return l8(v.xs + tok * kXStride + kb * 32 + 8 * ln.q);
-}
-
-// The per-type loops below are not unrolled (unrolling them makes the
-// compiler keep every iteration's MFMA results and operands live at once);
-// instead of indexing a register array with the loop counter (which would
-// move the array to scratch memory), each iteration uses element 0 and the
-// arrays are rotated by one at its end.
-template <int N>
-__device__ __forceinline__ void rotate(uint64_t (&a)[N]) {
-#pragma unroll
-  for (int i = 0; i + 1 < N; i++) a[i] = a[i + 1];
-}
-
-// ---- per-type weight fragments and term evaluation --------------------------
-template <uint32_t TY>
-struct GT;
-
-// Q4_K: lane k-range 8q..8q+7 of block 2g is the low nibbles of item bytes
-// 16 + 32g + 8q .. +8, of block 2g+1 their high nibbles. The row scales
-// d*sc and dmin*m (get_scale_min_k4, quant.rs:176-185) are staged once per
-// super-block for the block's 64 rows (stage_store), not decoded per lane.
+template <int MT>
+struct Vec;
 template <>
-struct GT<RLH_TYPE_Q4_K> {
-  static constexpr bool kNeedS = true;  // block sums and row scales staged
-  static constexpr bool kBlockMajor = true;
-  struct W {
-    uint64_t qs[4];
-  };
-  __device__ __forceinline__ static void load(W& r, const DevMat& w, uint32_t row, uint32_t j, uint32_t q) {
-    const ItemPtr p = item_ptr(w, row, j);
-#pragma unroll
-    for (int g = 0; g < 4; g++) r.qs[g] = g8(at(p, 16 + 32 * g + 8 * q));
-  }
-  __device__ __forceinline__ static void compute(const W (&w)[2], const StageView& v, const Lane& ln,
-                                                 float (&acc)[2][2][4]) {
-    const uint64_t m4 = 0x0F0F0F0F0F0F0F0Full;
-#pragma unroll 2
-    for (int g = 0; g < 4; g++) {
-      long alo[2], ahi[2];
-#pragma unroll
-      for (int tr = 0; tr < 2; tr++) {
-        alo[tr] = a_frag(v, ln, tr, 2 * g);
-        ahi[tr] = a_frag(v, ln, tr, 2 * g + 1);
-      }
-      f32x4_t rsc[2];  // {d1, mm1, d2, mm2} of the lane's rows
-      uint64_t blo[2], bhi[2];
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) {
-        const uint64_t qg = g == 0 ? w[tc].qs[0] : (g == 1 ? w[tc].qs[1] : (g == 2 ? w[tc].qs[2] : w[tc].qs[3]));
-        blo[tc] = qg & m4;
-        bhi[tc] = (qg >> 4) & m4;
-        rsc[tc] = v.rs[g * kTile + 32 * ln.rw + 16 * tc + ln.i16];
-      }
-#pragma unroll
-      for (int tr = 0; tr < 2; tr++) {
-        const f32x4_t da = tok4(v.d, ln, tr, 2 * g), db = tok4(v.d, ln, tr, 2 * g + 1);
-        const f32x4_t sa = tok4(v.s, ln, tr, 2 * g), sb = tok4(v.s, ln, tr, 2 * g + 1);
-#pragma unroll
-        for (int tc = 0; tc < 2; tc++) {
-          const v4i c1 = mfma(alo[tr], blo[tc]);
-          const v4i c2 = mfma(ahi[tr], bhi[tc]);
-          const float d1 = rsc[tc].x, mm1 = rsc[tc].y, d2 = rsc[tc].z, mm2 = rsc[tc].w;
-#pragma unroll
-          for (int e = 0; e < 4; e++)  // simd.rs:581
-            acc[tr][tc][e] = acc[tr][tc][e] + (da[e] * (d1 * (float)c1[e] - mm1 * sa[e]) +
-                                               db[e] * (d2 * (float)c2[e] - mm2 * sb[e]));
-        }
-      }
-    }
-  }
+struct Vec<32> {
+  typedef v16i I;
+  static constexpr int N = 16;
 };
-
-// Q6_K: block c of half h covers item bytes ql[64h + 32(c&1) + p] (nibble
-// c >> 1) and qh[128 + 32h + p] (bits 2c, 2c+1), p = position 0..31; the
-// lane's positions 8q..8q+7 all belong to sub-half s = q >> 1.
 template <>
-struct GT<RLH_TYPE_Q6_K> {
-  static constexpr bool kNeedS = false;
-  static constexpr bool kBlockMajor = false;  // four blocks of one token per read
-  struct W {
-    uint64_t ql[2][2], qh[2];
-    u32x4_t sc;
-    uint32_t d;
-  };
-  __device__ __forceinline__ static void load(W& r, const DevMat& w, uint32_t row, uint32_t j, uint32_t q) {
-    const ItemPtr p = item_ptr(w, row, j);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      r.ql[h][0] = g8(at(p, 64 * h + 8 * q));
-      r.ql[h][1] = g8(at(p, 64 * h + 32 + 8 * q));
-      r.qh[h] = g8(at(p, 128 + 32 * h + 8 * q));
-    }
-    r.sc = g16(at(p, 192));
-    r.d = ld_g2(p.tail);
-  }
-  __device__ __forceinline__ static void compute(const W (&w)[2], const StageView& v, const Lane& ln,
-                                                 float (&acc)[2][2][4]) {
-    const uint64_t m4 = 0x0F0F0F0F0F0F0F0Full, m2 = 0x0303030303030303ull;
-    const uint64_t hi = 0x8080808080808080ull, k32 = 0x2020202020202020ull;
-    const bool sub1 = ln.q >= 2;
-    uint64_t hq[2][4], hh[2][2];  // per row tile: ql pieces of half 0 then 1, qh of half 0 then 1
-    uint32_t hs[2][4];            // scale words of half 0 then 1
-#pragma unroll
-    for (int tc = 0; tc < 2; tc++) {
-      hq[tc][0] = w[tc].ql[0][0];
-      hq[tc][1] = w[tc].ql[0][1];
-      hq[tc][2] = w[tc].ql[1][0];
-      hq[tc][3] = w[tc].ql[1][1];
-      hh[tc][0] = w[tc].qh[0];
-      hh[tc][1] = w[tc].qh[1];
-      hs[tc][0] = w[tc].sc.x;
-      hs[tc][1] = w[tc].sc.y;
-      hs[tc][2] = w[tc].sc.z;
-      hs[tc][3] = w[tc].sc.w;
-    }
-#pragma unroll 1
-    for (int h = 0; h < 2; h++) {
-      // signed weights q = u - 32 of the half's 4 blocks, per row tile
-      uint64_t bq[2][4];
-      float dsc[2][2][4];
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) {
-        const float d = f16_to_f32(w[tc].d);
-        const uint32_t swlo = hs[tc][0], swhi = hs[tc][1];  // the half's 8 scales
-        const uint64_t ql0 = hq[tc][0], ql1 = hq[tc][1], qh = hh[tc][0];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const uint64_t nib = (((c & 1) ? ql1 : ql0) >> (4 * (c >> 1))) & m4;
-          const uint64_t u = nib | (((qh >> (2 * c)) & m2) << 4);
-          bq[tc][c] = ((u | hi) - k32) ^ hi;
-#pragma unroll
-          for (int s = 0; s < 2; s++) {
-            const uint32_t bi = s + 2 * c;  // scales[sub + 2c] of the half (simd.rs:626-629)
-            dsc[tc][s][c] = d * (float)(int8_t)(((bi < 4 ? swlo : swhi) >> (8 * (bi & 3))) & 0xff);
-          }
-        }
-      }
-      long a[2][4];
-      f32x4_t da[2][4];  // [tr][e] -> da of blocks 4h..4h+3 (token-major staging)
-#pragma unroll
-      for (int tr = 0; tr < 2; tr++) {
-#pragma unroll
-        for (int c = 0; c < 4; c++) a[tr][c] = a_frag(v, ln, tr, 4 * h + c);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const uint32_t tok = 32 * ln.tw + 16 * tr + 4 * ln.q + e;
-          da[tr][e] = *(const RLH_LDS f32x4_t*)(v.d + tok * 8 + 4 * h);
-        }
-      }
-      // terms in the order s = 0 (c = 0..3), then s = 1 (simd.rs:630-665);
-      // the four products of a (s, c) step are issued before their
-      // combines, so no combine waits on the product just issued
-#pragma unroll
-      for (int s = 0; s < 2; s++) {
-        const bool keep = (s == 1) == sub1;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          v4i ci[2][2];
-#pragma unroll
-          for (int tr = 0; tr < 2; tr++)
-#pragma unroll
-            for (int tc = 0; tc < 2; tc++) ci[tr][tc] = mfma(a[tr][c], keep ? bq[tc][c] : 0ull);
-#pragma unroll
-          for (int tr = 0; tr < 2; tr++) {
-#pragma unroll
-            for (int tc = 0; tc < 2; tc++) {
-#pragma unroll
-              for (int e = 0; e < 4; e++)  // simd.rs:663
-                acc[tr][tc][e] = acc[tr][tc][e] + dsc[tc][s][c] * (float)ci[tr][tc][e] * da[tr][e][c];
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) {  // half 1 moves into place
-        hq[tc][0] = hq[tc][2];
-        hq[tc][1] = hq[tc][3];
-        hh[tc][0] = hh[tc][1];
-        hs[tc][0] = hs[tc][2];
-        hs[tc][1] = hs[tc][3];
-      }
-    }
-  }
+struct Vec<16> {
+  typedef v4i I;
+  static constexpr int N = 4;
 };
 
-// Q8_0: item = 8 blocks; lane bytes 32k + 8q .. +8 of block k, then the 8
-// f16 scales at item bytes 256..271.
-template <>
-struct GT<RLH_TYPE_Q8_0> {
-  static constexpr bool kNeedS = false;
-  static constexpr bool kBlockMajor = true;
-  struct W {
-    uint64_t qs[8];
-    u32x4_t dv;
-  };
-  __device__ __forceinline__ static void load(W& r, const DevMat& w, uint32_t row, uint32_t j, uint32_t q) {
-    const ItemPtr p = item_ptr(w, row, j);
+__device__ __forceinline__ uint64_t l8(const lbyte* p) { return *(const RLH_LDS uint64_t*)p; }
+__device__ __forceinline__ float ub(uint32_t w, int b) { return (float)((w >> (8 * b)) & 0xffu); }
+
+// The steps of a combine over N elements. N = 16: every step over 8 elements
+// before the next one, since an f32 add or multiply issues every 4.6 cycles
+// from one wave but its result takes 9, and a chain written element by
+// element (the order the compiler's scheduler prefers, to save registers)
+// runs at half rate. N = 4: left to the scheduler, which has the registers
+// to overlap blocks.
+template <int N, class... F>
+__device__ __forceinline__ void phases(F... f) {
+  constexpr int M = N < 8 ? N : 8;
 #pragma unroll
-    for (int k = 0; k < 8; k++) r.qs[k] = g8(at(p, 32 * k + 8 * q));
-    r.dv = g16(at(p, 256));
+  for (int e0 = 0; e0 < N; e0 += M) {
+    auto step = [&](auto g) {
+#pragma unroll
+      for (int e = e0; e < e0 + M; e++) g(e);
+      if constexpr (N > 8) __builtin_amdgcn_sched_barrier(0);
+    };
+    (step(f), ...);
   }
-  __device__ __forceinline__ static void compute(const W (&wr)[2], const StageView& v, const Lane& ln,
-                                                 float (&acc)[2][2][4]) {
-    uint64_t qs[2][8];
-    uint32_t dw[2][4];
+}
+
+// A wave's place in its block and the LDS views of the current stage.
+template <uint32_t TY, int MT>
+struct Wave {
+  using G = Geo<TY, MT>;
+  static constexpr int N = Vec<MT>::N;
+  uint32_t lane, l, q;  // q: lane group (MT 32: half 0/1; MT 16: 0..3)
+  uint32_t tw, rw;
+  const lbyte* qs;
+  const lbyte* ds;
+  const lbyte* w;
+  const lbyte* tail;
+  __device__ __forceinline__ void view(const lbyte* buf) {
+    qs = buf + (MT == 32 ? tw * 4096u : 0u);
+    ds = buf + G::kDOff + (MT == 32 ? tw * 512u : 0u);
+    w = buf + G::kWOff;
+    tail = buf + G::kTailOff;
+  }
+  // row of the block that the lane holds
+  __device__ __forceinline__ uint32_t row() const { return rw * MT + l; }
+  // scales of the lane's N tokens for block kb: element e = 4 g + i is token
+  // 8 g + 4 q + i (MT 32) or 16 tw + 4 q + i (MT 16)
+  __device__ __forceinline__ void scales(float (&d)[N], uint32_t kb) const {
+    const RLH_LDS float* b = (const RLH_LDS float*)ds + kb * 32 + 4 * q + (MT == 16 ? 16 * tw : 0u);
 #pragma unroll
-    for (int tc = 0; tc < 2; tc++) {
+    for (int g = 0; g < N / 4; g++) {
+      const f32x4_t v = *(const RLH_LDS f32x4_t*)(b + 8 * g);
 #pragma unroll
-      for (int k = 0; k < 8; k++) qs[tc][k] = wr[tc].qs[k];
-      dw[tc][0] = wr[tc].dv.x;
-      dw[tc][1] = wr[tc].dv.y;
-      dw[tc][2] = wr[tc].dv.z;
-      dw[tc][3] = wr[tc].dv.w;
-    }
-#pragma unroll 2
-    for (int k = 0; k < 8; k++) {
-      float dk[2];
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) dk[tc] = f16_to_f32((dw[tc][0] >> (16 * (k & 1))) & 0xffff);
-#pragma unroll
-      for (int tr = 0; tr < 2; tr++) {
-        const long a = a_frag(v, ln, tr, k);
-        const f32x4_t da = tok4(v.d, ln, tr, k);
-#pragma unroll
-        for (int tc = 0; tc < 2; tc++) {
-          const v4i ci = mfma(a, qs[tc][0]);
-#pragma unroll
-          for (int e = 0; e < 4; e++)  // simd.rs:891
-            acc[tr][tc][e] = acc[tr][tc][e] + dk[tc] * (float)ci[e] * da[e];
-        }
-      }
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) {
-        rotate(qs[tc]);
-        if (k & 1) {  // next pair of f16 scales
-          dw[tc][0] = dw[tc][1];
-          dw[tc][1] = dw[tc][2];
-          dw[tc][2] = dw[tc][3];
-        }
-      }
+      for (int i = 0; i < 4; i++) d[4 * g + i] = v[i];
     }
   }
-};
-
-// Q4_0: item = 8 blocks of 16 bytes; positions 0..15 are the low nibbles,
-// 16..31 the high nibbles, so lane q reads bytes 16k + 8(q & 1) .. +8 and
-// takes nibble q >> 1; weights are nibble - 8.
-template <>
-struct GT<RLH_TYPE_Q4_0> {
-  static constexpr bool kNeedS = false;
-  static constexpr bool kBlockMajor = true;
-  struct W {
-    uint64_t qs[8];
-    u32x4_t dv;
-  };
-  __device__ __forceinline__ static void load(W& r, const DevMat& w, uint32_t row, uint32_t j, uint32_t q) {
-    const ItemPtr p = item_ptr(w, row, j);
+  // the scales of elements e .. e + 3 (e a multiple of 4) into d[e & 7] ..
+  __device__ __forceinline__ void scale8(float (&d)[8], uint32_t kb, int e) const {
+    if (e & 3) return;
+    const f32x4_t x = *(const RLH_LDS f32x4_t*)((const RLH_LDS float*)ds + kb * 32 + 4 * q +
+                                                (MT == 16 ? 16 * tw : 0u) + 2 * e);
 #pragma unroll
-    for (int k = 0; k < 8; k++) r.qs[k] = g8(at(p, 16 * k + 8 * (q & 1)));
-    r.dv = g16(at(p, 128));
+    for (int i = 0; i < 4; i++) d[(e & 7) + i] = x[i];
   }
-  __device__ __forceinline__ static void compute(const W (&wr)[2], const StageView& v, const Lane& ln,
-                                                 float (&acc)[2][2][4]) {
-    const uint64_t m4 = 0x0F0F0F0F0F0F0F0Full, hi = 0x8080808080808080ull, k8 = 0x0808080808080808ull;
-    uint64_t qs[2][8];
-    uint32_t dw[2][4];
-#pragma unroll
-    for (int tc = 0; tc < 2; tc++) {
-#pragma unroll
-      for (int k = 0; k < 8; k++) qs[tc][k] = wr[tc].qs[k];
-      dw[tc][0] = wr[tc].dv.x;
-      dw[tc][1] = wr[tc].dv.y;
-      dw[tc][2] = wr[tc].dv.z;
-      dw[tc][3] = wr[tc].dv.w;
-    }
-#pragma unroll 2
-    for (int k = 0; k < 8; k++) {
-      float dk[2];
-      uint64_t b[2];
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) {
-        dk[tc] = f16_to_f32((dw[tc][0] >> (16 * (k & 1))) & 0xffff);
-        const uint64_t nib = (qs[tc][0] >> (4 * (ln.q >> 1))) & m4;
-        b[tc] = ((nib | hi) - k8) ^ hi;
-      }
-#pragma unroll
-      for (int tr = 0; tr < 2; tr++) {
-        const long a = a_frag(v, ln, tr, k);
-        const f32x4_t da = tok4(v.d, ln, tr, k);
-#pragma unroll
-        for (int tc = 0; tc < 2; tc++) {
-          const v4i ci = mfma(a, b[tc]);
-#pragma unroll
-          for (int e = 0; e < 4; e++)  // simd.rs:863
-            acc[tr][tc][e] = acc[tr][tc][e] + dk[tc] * (float)ci[e] * da[e];
-        }
-      }
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) {
-        rotate(qs[tc]);
-        if (k & 1) {
-          dw[tc][0] = dw[tc][1];
-          dw[tc][1] = dw[tc][2];
-          dw[tc][2] = dw[tc][3];
-        }
-      }
-    }
+  // sum of the quants of block kb of one token per lane: token l (MT 32, its
+  // tile) or 16 tw + l (MT 16)
+  __device__ __forceinline__ float sum(uint32_t kb) const {
+    const RLH_LDS int32_t* b = (const RLH_LDS int32_t*)(ds + 512 * G::kActTiles);
+    return (float)b[kb * 32 + (MT == 16 ? 16 * tw : 0u) + l];
   }
-};
-
-// Stages super-block j of the block's 64 tokens: Q8 bytes into the padded
-// [64][272] layout (17 slots of 16 bytes per token, the 17th unused), the 8
-// block scales of every token, and for Q4_K the 8 block sums (as f32) and the
-// 64 rows' scale headers turned into {d*sc, dmin*m} pairs. Scales and sums
-// are stored block-major ([block][token]) for the types that read them four
-// tokens at a time (Q4_K, Q8_0, Q4_0), token-major for Q6_K (four blocks of
-// one token at a time). The copy goes through registers: stage_load issues
-// the global loads at the top of a super-block step and stage_store writes
-// them to LDS at its end, so their latency hides behind the step's products.
-// (Copies straight into LDS, global_load_lds, measured ~0.5 us per
-// instruction per wave here: the step's copies took as long as its
-// products.) Jobs of thread t, wave w = t / 64 (every role is whole waves,
-// so the branches are uniform): jobs 0-3 Q8 slots t + 256k; job 4 Q8 slots
-// 1024-1087 (wave 0), the scales (waves 1-2: 128 slots of 16 bytes, token
-// (t - 64) / 2, blocks 4 ((t - 64) & 1) .. +3), the sums of tokens 0-31
-// (wave 3, Q4_K); job 5 (Q4_K) the sums of tokens 32-63 (wave 0) and the
-// row headers (wave 1). Slots past the valid tokens or the 17th slot of a
-// token load a clamped, valid address and are not stored.
-constexpr uint32_t kStageJobs = 6;
-
-struct StageRegs {
-  u32x4_t v[kStageJobs];
-  const uint8_t* src[kStageJobs];  // job k's source for the current super-block (not the header job)
-  uint32_t keep;                   // bit k: job k is stored
-  uint32_t sub4, sub5;             // jobs 4/5: scale or sum slot (token * 2 + half), or the header row
-};
-
-__device__ __forceinline__ uint32_t wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
-
-// Sources of super-block 0; super-block j + 1 is 256 bytes further for Q8
-// bytes and 32 bytes for scales and sums; the header job addresses item
-// (row, j) itself.
-__device__ __forceinline__ void stage_init(StageRegs& r, const GemmArgs& a, uint32_t t0, bool q4k) {
-  const uint32_t cols = a.w.cols, nb = cols / 32, t = threadIdx.x, w = wave_id();
-  r.keep = 0;
-  auto q8_job = [&](uint32_t k, uint32_t p) {
-    const uint32_t tok = p / 17, ch = p - tok * 17;
-    r.keep |= (ch < 16 && t0 + tok < a.n) ? 1u << k : 0u;
-    r.src[k] = (const uint8_t*)a.x.qs + (size_t)min(t0 + tok, a.n - 1) * cols + 16 * min(ch, 15u);
-  };
-  auto small_job = [&](uint32_t k, const void* base, uint32_t slot) {
-    const uint32_t tok = slot >> 1;
-    r.keep |= t0 + tok < a.n ? 1u << k : 0u;
-    r.src[k] = (const uint8_t*)base + ((size_t)min(t0 + tok, a.n - 1) * nb + 4 * (slot & 1)) * 4;
-  };
-#pragma unroll
-  for (uint32_t k = 0; k < 4; k++) q8_job(k, t + 256 * k);
-  r.sub4 = r.sub5 = 0;
-  r.src[4] = r.src[5] = (const uint8_t*)a.x.d;
-  if (w == 0) {
-    q8_job(4, t + 1024);
-  } else if (w <= 2) {
-    r.sub4 = t - 64;
-    small_job(4, a.x.d, r.sub4);
-  } else if (q4k) {
-    r.sub4 = t - 192;
-    small_job(4, a.x.s, r.sub4);
-  }
-  if (q4k && w == 0) {
-    r.sub5 = t + 64;
-    small_job(5, a.x.s, r.sub5);
-  } else if (q4k && w == 1) {
-    r.sub5 = t - 64;
-    r.keep |= 1u << 5;
-  }
-}
-
-// q8_dma: the Q8 byte jobs (0..3, and job 4 of wave 0) go by DMA
-// (stage_dma_q8) and are skipped here.
-__device__ __forceinline__ void stage_load(StageRegs& r, const GemmArgs& a, uint32_t row0, uint32_t j, bool q4k,
-                                           bool q8_dma = false) {
-  const uint32_t w = wave_id();
-#pragma unroll
-  for (uint32_t k = 0; k < 5; k++) {
-    if (q8_dma && (k < 4 || w == 0)) continue;
-    r.v[k] = *(const RLH_GLOBAL u32x4_t*)r.src[k];
-    r.src[k] += (k < 4 || w == 0) ? 256 : 32;
-  }
-  if (q4k && w == 0) {
-    r.v[5] = *(const RLH_GLOBAL u32x4_t*)r.src[5];
-    r.src[5] += 32;
-  } else if (q4k && w == 1) {  // the row's d, dmin and 12 scale bytes (item bytes 0..15)
-    r.v[5] = *(const RLH_GLOBAL u32x4_t*)item_ptr(a.w, min(row0 + r.sub5, a.w.rows - 1), j).base;
-  }
-}
-
-// Q6_K stages super-block j by DMA straight into `buf` (global_load_lds, 16
-// bytes per lane; no staging registers): the 64 tokens' Q8 bytes (1088
-// pieces of 16 bytes, token p / 17, piece p % 17; the pad piece repeats
-// piece 15 and tokens past n repeat the last one, neither is read for a
-// kept output) and the token-major block scales (128 slots of 16 bytes).
-// Every wave issues its copies; the caller waits for them (vmcnt) and then
-// the block barrier.
-__device__ __forceinline__ void stage_dma_q8(const GemmArgs& a, uint32_t t0, uint32_t j, lbyte* buf) {
-  const uint32_t cols = a.w.cols, lane = threadIdx.x & 63, w = wave_id();
-  auto q8_piece = [&](uint32_t p0) {  // pieces p0 .. p0 + 63, p0 a multiple of 64
-    const uint32_t p = p0 + lane, tok = p / 17, ch = p - tok * 17;
-    const int8_t* src = a.x.qs + (size_t)min(t0 + tok, a.n - 1) * cols + 256 * j + 16 * min(ch, 15u);
-    __builtin_amdgcn_global_load_lds((const RLH_GLOBAL void*)src, (RLH_LDS void*)(buf + p0 * 16), 16, 0, 0);
-  };
-#pragma unroll
-  for (uint32_t k = 0; k < 4; k++) q8_piece(64 * w + 256 * k);
-  if (w == 0) q8_piece(1024);
-}
-__device__ __forceinline__ void stage_dma(const GemmArgs& a, uint32_t t0, uint32_t j, lbyte* buf) {
-  const uint32_t nb = a.w.cols / 32, lane = threadIdx.x & 63, w = wave_id();
-  stage_dma_q8(a, t0, j, buf);
-  if (w == 1 || w == 2) {  // scale slots (token slot >> 1, blocks 4 (slot & 1) .. +3)
-    const uint32_t slot = 64 * (w - 1) + lane, tok = slot >> 1;
-    const float* src = a.x.d + (size_t)min(t0 + tok, a.n - 1) * nb + 8 * j + 4 * (slot & 1);
-    __builtin_amdgcn_global_load_lds((const RLH_GLOBAL void*)src,
-                                     (RLH_LDS void*)(buf + kXBytes + 4 * 64 * (w - 1) * 4), 16, 0, 0);
-  }
-}
-
-// A scale or sum slot (token slot >> 1, blocks 4 (slot & 1) .. +3) into LDS.
-__device__ __forceinline__ void store_small(lbyte* buf, bool sum, bool block_major, uint32_t slot, const u32x4_t& v) {
-  RLH_LDS float* base = (RLH_LDS float*)(buf + kXBytes + (sum ? kDBytes : 0u));
-  const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-  if (block_major) {
-    RLH_LDS float* t = base + 4 * (slot & 1) * kTile + (slot >> 1);
-#pragma unroll
-    for (int i = 0; i < 4; i++) t[i * kTile] = sum ? (float)(int32_t)w4[i] : __uint_as_float(w4[i]);
-  } else {
-    *(RLH_LDS u32x4_t*)(base + 4 * slot) = v;
-  }
-}
-
-template <bool kBlockMajor>
-__device__ __forceinline__ void stage_store(const StageRegs& r, lbyte* buf, bool q4k, bool q8_dma = false) {
-  const uint32_t t = threadIdx.x, w = wave_id();
-  if (!q8_dma) {
-#pragma unroll
-    for (uint32_t k = 0; k < 4; k++)
-      if (r.keep >> k & 1u) *(RLH_LDS u32x4_t*)(buf + (t + 256 * k) * 16) = r.v[k];
-  }
-  if (r.keep >> 4 & 1u) {
-    if (w == 0) {
-      if (!q8_dma) *(RLH_LDS u32x4_t*)(buf + (t + 1024) * 16) = r.v[4];
+  // 16 bytes (MT 32) or 8 (MT 16) of the token operand of block kb; the
+  // weight operand (wfrag) takes the same positions in the same order
+  __device__ __forceinline__ v4i afrag(uint32_t kb) const {
+    if constexpr (MT == 32) {
+      return *(const RLH_LDS v4i*)(qs + kb * 1024 + lane * 16);
     } else {
-      store_small(buf, w == 3, kBlockMajor, r.sub4, r.v[4]);
+      const uint64_t x = l8(qs + kb * 1024 + (q & 1) * 512 + (16 * tw + l) * 16 + (q >> 1) * 8);
+      return v4i{(int)(uint32_t)x, (int)(uint32_t)(x >> 32), 0, 0};
     }
   }
-  if (q4k && (r.keep >> 5 & 1u)) {
-    if (w == 0) {
-      store_small(buf, true, kBlockMajor, r.sub5, r.v[5]);
+  __device__ __forceinline__ const lbyte* chunk(uint32_t c) const { return w + (c * G::kRows + row()) * 16; }
+  // bytes of a 32-value run stored one byte per value in chunks c0, c0 + 1
+  __device__ __forceinline__ v4i wfrag(uint32_t c0) const {
+    if constexpr (MT == 32) {
+      const uint64_t x = l8(chunk(c0) + 8 * q), y = l8(chunk(c0 + 1) + 8 * q);
+      return v4i{(int)(uint32_t)x, (int)(uint32_t)(x >> 32), (int)(uint32_t)y, (int)(uint32_t)(y >> 32)};
     } else {
-      // get_scale_min_k4 (quant.rs:176-185) of the 8 sub-blocks; the pairs
-      // d*sc, dmin*m of sub-blocks 2g, 2g+1 (exact in f32: an f16 times a
-      // 6-bit integer)
-      const u32x4_t v = r.v[5];
-      RLH_LDS f32x4_t* rs = (RLH_LDS f32x4_t*)(buf + kXBytes + 2 * kDBytes);
-      const float dd = f16_to_f32(v.x & 0xffff), dmin = f16_to_f32(v.x >> 16);
-      const uint32_t s0 = v.y, s1 = v.z, s2 = v.w;
+      const uint64_t x = l8(chunk(c0 + (q >> 1)) + 8 * (q & 1));
+      return v4i{(int)(uint32_t)x, (int)(uint32_t)(x >> 32), 0, 0};
+    }
+  }
+  __device__ __forceinline__ static typename Vec<MT>::I base() {
+    typename Vec<MT>::I m;
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        uint32_t sc[2], m[2];
+    for (int i = 0; i < N; i++) m[i] = kBase;
+    return m;
+  }
+  // kBase + the dots of a 32-value block
+  __device__ __forceinline__ static typename Vec<MT>::I dot32(v4i a, v4i b) {
+    if constexpr (MT == 32)
+      return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, base(), 0, 0, 0);
+    else
+      return __builtin_amdgcn_mfma_i32_16x16x32_i8(lo64(a), lo64(b), base(), 0, 0, 0);
+  }
+  // kBase + the dots of a 16-value half of a block (MT 32: each lane's 8
+  // bytes of it; MT 16: lane groups 2s, 2s + 1 hold half s, the others'
+  // weights are zero)
+  __device__ __forceinline__ static typename Vec<MT>::I dot16(uint64_t a, uint64_t b) {
+    if constexpr (MT == 32)
+      return __builtin_amdgcn_mfma_i32_32x32x16_i8((long)a, (long)b, base(), 0, 0, 0);
+    else
+      return __builtin_amdgcn_mfma_i32_16x16x32_i8((long)a, (long)b, base(), 0, 0, 0);
+  }
+  __device__ __forceinline__ static long lo64(v4i v) { return (long)(((uint64_t)(uint32_t)v.y << 32) | (uint32_t)v.x); }
+  // the dot in units of 2^-26
+  __device__ __forceinline__ static float dotf(int c) { return __int_as_float(c) - kBaseF; }
+};
+
+// ---- half a super-block of a wave, per type ---------------------------------
+// acc[e]: the lane's row, its e-th token; h = the half.
+template <uint32_t TY, int MT>
+struct Step;
+
+// Q4_K: staged chunk 0 = d, dmin, 12 scale bytes; chunks 1 + 2g, 2 + 2g hold
+// block 2g of the half in the low and 2g + 1 in the high nibbles.
+template <int MT>
+struct Step<RLH_TYPE_Q4_K, MT> {
+  using W = Wave<RLH_TYPE_Q4_K, MT>;
+  static constexpr int N = W::N;
+  __device__ __forceinline__ static void run(const W& v, uint32_t h, float (&acc)[N]) {
+    const u32x4_t hd = *(const RLH_LDS u32x4_t*)v.chunk(0);
+    const float d = kUnit * f16_to_f32(hd.x & 0xffff), dmin = f16_to_f32(hd.x >> 16);
+    // get_scale_min_k4 (quant.rs:176-185): the half's four 6-bit values of each kind
+    const uint32_t sc = h ? (hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u) : hd.y & 0x3F3F3F3Fu;
+    uint32_t mn = h ? ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u) : hd.z & 0x3F3F3F3Fu;
+    mn >>= 8 * v.q;  // the lane group's own block of a rank-1 product in byte 0 (and 2)
+    f32x16_t pm;     // MT 16: the half's four rank-1 products
+    if constexpr (MT == 16)
+      pm = __builtin_amdgcn_mfma_f32_16x16x1f32(v.sum(v.q), dmin * ub(mn, 0), f32x16_t{}, 0, 0, 0);
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const uint32_t sh = 16 * (g & 1) + 8 * h;
-          if (g < 2) {
-            sc[h] = (s0 >> sh) & 63;
-            m[h] = (s1 >> sh) & 63;
-          } else {
-            sc[h] = ((s2 >> sh) & 0xF) | (((s0 >> sh) >> 6 & 3) << 4);
-            m[h] = ((s2 >> sh) >> 4 & 0xF) | (((s1 >> sh) >> 6 & 3) << 4);
-          }
-        }
-        rs[g * kTile + r.sub5] = f32x4_t{dd * (float)sc[0], dmin * (float)m[0], dd * (float)sc[1], dmin * (float)m[1]};
+    for (int g = 0; g < 2; g++) {
+      const v4i a0 = v.afrag(2 * g), a1 = v.afrag(2 * g + 1), x = v.wfrag(1 + 2 * g);
+      v4i b0, b1;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        b0[i] = x[i] & 0x0F0F0F0F;
+        b1[i] = (int)(((uint32_t)x[i] >> 4) & 0x0F0F0F0Fu);
+      }
+      const float d0 = d * ub(sc, 2 * g), d1 = d * ub(sc, 2 * g + 1);
+      float p0[N], p1[N];  // dmin*m * sum, each rounded once
+      if constexpr (MT == 32) {
+        const f32x32_t p =
+            __builtin_amdgcn_mfma_f32_32x32x1f32(v.sum(2 * g + v.q), dmin * ub(mn, 2 * g), f32x32_t{}, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < N; e++) p0[e] = p[e], p1[e] = p[N + e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < N; e++) p0[e] = pm[8 * g + e], p1[e] = pm[8 * g + 4 + e];
+      }
+      // acc + (da * (d0 * dot0 - p0) + db * (d1 * dot1 - p1)) (simd.rs:581),
+      // one block after the other and the scales eight at a time: the wave
+      // stays within 128 registers
+      float f0[N], f1[N], sc8[8];
+      const auto c0 = W::dot32(a0, b0);
+      phases<N>([&](int e) { v.scale8(sc8, 2 * g, e); }, [&](int e) { f0[e] = W::dotf(c0[e]); },
+                [&](int e) { f0[e] = d0 * f0[e]; }, [&](int e) { f0[e] = f0[e] - p0[e]; },
+                [&](int e) { f0[e] = sc8[e & 7] * f0[e]; });
+      const auto c1 = W::dot32(a1, b1);
+      phases<N>([&](int e) { v.scale8(sc8, 2 * g + 1, e); }, [&](int e) { f1[e] = W::dotf(c1[e]); },
+                [&](int e) { f1[e] = d1 * f1[e]; }, [&](int e) { f1[e] = f1[e] - p1[e]; },
+                [&](int e) { f1[e] = sc8[e & 7] * f1[e]; }, [&](int e) { f0[e] = f0[e] + f1[e]; },
+                [&](int e) { acc[e] = acc[e] + f0[e]; });
+    }
+  }
+};
+
+// Q6_K: block c of the half is the nibbles c >> 1 of staged chunks 2 (c & 1)
+// .. + 1 and bits 2c, 2c + 1 of chunks 4, 5; chunk 6 = 16 scales.
+template <int MT>
+struct Step<RLH_TYPE_Q6_K, MT> {
+  using W = Wave<RLH_TYPE_Q6_K, MT>;
+  static constexpr int N = W::N;
+  // the lane's bytes of 16-value half s of chunk pair c0 (MT 16: lane groups
+  // 2s, 2s + 1 hold half s, whatever s is asked for)
+  __device__ __forceinline__ static uint64_t raw(const W& v, uint32_t c0, int s) {
+    return MT == 32 ? l8(v.chunk(c0 + s) + 8 * v.q) : l8(v.chunk(c0 + (v.q >> 1)) + 8 * (v.q & 1));
+  }
+  // 4 (u - 32) of the four blocks: the six bits at the top of the byte, the
+  // sign bit flipped
+  __device__ __forceinline__ static void weights(const W& v, int s, uint64_t (&b)[4]) {
+    const uint64_t x0 = raw(v, 0, s), x1 = raw(v, 2, s), f = raw(v, 4, s) ^ 0xAAAAAAAAAAAAAAAAull;
+    const uint32_t w0[2] = {(uint32_t)x0, (uint32_t)(x0 >> 32)}, w1[2] = {(uint32_t)x1, (uint32_t)(x1 >> 32)};
+    const uint32_t wf[2] = {(uint32_t)f, (uint32_t)(f >> 32)};
+    uint32_t o[4][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      o[0][i] = ((w0[i] << 2) & 0x3C3C3C3Cu) | ((wf[i] << 6) & 0xC0C0C0C0u);
+      o[1][i] = ((w1[i] << 2) & 0x3C3C3C3Cu) | ((wf[i] << 4) & 0xC0C0C0C0u);
+      o[2][i] = ((w0[i] >> 2) & 0x3C3C3C3Cu) | ((wf[i] << 2) & 0xC0C0C0C0u);
+      o[3][i] = ((w1[i] >> 2) & 0x3C3C3C3Cu) | (wf[i] & 0xC0C0C0C0u);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) b[c] = ((uint64_t)o[c][1] << 32) | o[c][0];
+  }
+  __device__ __forceinline__ static void run(const W& v, uint32_t h, float (&acc)[N]) {
+    // the row's f16 in its 4-byte word (even rows low, odd rows high); the
+    // weights enter as 4 q
+    const uint32_t r = v.row();
+    const float dq = 0.25f * kUnit *
+                     f16_to_f32((*(const RLH_LDS uint32_t*)(v.tail + 4 * r) >> (16 * (r & 1))) & 0xffff);
+    const uint64_t sw = l8(v.chunk(6) + 8 * h);  // the half's 8 scales
+    uint64_t all[4];
+    if constexpr (MT == 16) weights(v, 0, all);
+    // terms in the order s = 0 (c = 0..3), then s = 1 (simd.rs:630-665)
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      uint64_t b[4];
+      if constexpr (MT == 32) {
+        weights(v, s, b);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; c++) b[c] = (v.q >> 1) == (uint32_t)s ? all[c] : 0;
+      }
+      uint64_t a[2];  // the operand and scales of block c + 1 are read while block c is combined
+      float da[2][N];
+      auto read = [&](int c) {
+        if constexpr (MT == 32)
+          a[c & 1] = l8(v.qs + c * 1024 + v.lane * 16 + 8 * s);
+        else
+          a[c & 1] = (uint64_t)W::lo64(v.afrag(c));
+        v.scales(da[c & 1], c);
+      };
+      read(0);
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        if (c < 3) read(c + 1);
+        const auto ci = W::dot16(a[c & 1], b[c]);
+        const float ds = dq * (float)(int8_t)(sw >> (8 * (s + 2 * c)));  // scales[s + 2c] (simd.rs:626-629)
+        float f[N];  // acc + (ds * dot) * da (simd.rs:663)
+        phases<N>([&](int e) { f[e] = W::dotf(ci[e]); }, [&](int e) { f[e] = ds * f[e]; },
+                  [&](int e) { f[e] = f[e] * da[c & 1][e]; }, [&](int e) { acc[e] = acc[e] + f[e]; });
       }
     }
   }
-}
+};
 
-// Q4_K fits 166 VGPRs when asked for three waves per SIMD (no scratch), so a
-// CU holds three of its blocks (3 x 51 KB of LDS); the other types keep the
-// allocator's choice.
-template <uint32_t TY>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TY == RLH_TYPE_Q4_K ? 3 : 1)))
-k_gemm(GemmArgs a0) {
-  using G = GT<TY>;
+// Q8_0: staged chunks 2k, 2k + 1 hold block k of the half, chunk 8 the 8 f16
+// scales. Q4_0: chunk k holds block k (positions 0..15 low nibbles, 16..31
+// high), chunk 4 the 8 f16 scales; the weights enter as 16 (nibble - 8).
+template <uint32_t TY, int MT>
+struct Step8 {
+  using W = Wave<TY, MT>;
+  static constexpr int N = W::N;
+  __device__ __forceinline__ static v4i weights(const W& v, uint32_t k) {
+    if constexpr (TY == RLH_TYPE_Q8_0) {
+      return v.wfrag(2 * k);
+    } else {
+      const uint64_t x = l8(v.chunk(k) + 8 * (MT == 32 ? v.q : (v.q & 1)));
+      const uint32_t w0 = (uint32_t)x, w1 = (uint32_t)(x >> 32), m = 0xF0F0F0F0u, f = 0x80808080u;
+      const v4i lo = {(int)(((w0 << 4) & m) ^ f), (int)(((w1 << 4) & m) ^ f), 0, 0};
+      const v4i hi = {(int)((w0 & m) ^ f), (int)((w1 & m) ^ f), 0, 0};
+      if constexpr (MT == 32) return v4i{lo.x, lo.y, hi.x, hi.y};
+      return (v.q >> 1) ? hi : lo;
+    }
+  }
+  __device__ __forceinline__ static void run(const W& v, uint32_t h, float (&acc)[N]) {
+    constexpr float kS = TY == RLH_TYPE_Q8_0 ? kUnit : 0.0625f * kUnit;
+    const uint64_t dv = l8(v.chunk(TY == RLH_TYPE_Q8_0 ? 8 : 4) + 8 * h);  // the half's four f16 scales
+    v4i a[2], b[2];  // the operands and scales of block k + 1 are read while block k is combined
+    float da[2][N];
+    auto read = [&](int k) {
+      a[k & 1] = v.afrag(k);
+      b[k & 1] = weights(v, k);
+      v.scales(da[k & 1], k);
+    };
+    read(0);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (k < 3) read(k + 1);
+      const auto ci = W::dot32(a[k & 1], b[k & 1]);
+      const float dk = kS * f16_to_f32((uint32_t)(dv >> (16 * k)) & 0xffff);
+      float f[N];  // acc + (dk * dot) * da (simd.rs:891, 863)
+      phases<N>([&](int e) { f[e] = W::dotf(ci[e]); }, [&](int e) { f[e] = dk * f[e]; },
+                [&](int e) { f[e] = f[e] * da[k & 1][e]; }, [&](int e) { acc[e] = acc[e] + f[e]; });
+    }
+  }
+};
+template <int MT>
+struct Step<RLH_TYPE_Q8_0, MT> : Step8<RLH_TYPE_Q8_0, MT> {};
+template <int MT>
+struct Step<RLH_TYPE_Q4_0, MT> : Step8<RLH_TYPE_Q4_0, MT> {};
+
+// Block b runs on XCD b % 8; the blocks of one XCD walk the token tiles of a
+// row tile first, so each weight tile is fetched into that XCD's L2 once and
+// reused by all token tiles.
+template <uint32_t TY, int MT>
+__global__ void __launch_bounds__(256, 4) k_gemm(GemmArgs a0) {
+  using G = Geo<TY, MT>;
+  using V = Wave<TY, MT>;
+  constexpr int N = V::N;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_generic[];
   lbyte* lds = (lbyte*)lds_generic;
-  // XCD-aware tile order (see file header)
   const uint32_t b = blockIdx.x, xcd = b & 7, k = b >> 3;
   const uint32_t tt = k % a0.n_tt, rtg = (k / a0.n_tt) * 8 + xcd;
   if (rtg >= a0.n_rt) return;  // whole block, before any barrier
   // the block's segment (uniform: from the block index)
-  GemmArgs a = a0;
+  DevMat w = a0.w;
+  float *y = a0.y, *resid = a0.resid;
   uint32_t rt = rtg;
   if (rtg >= a0.n_rt1) {
-    a.w = a0.w2;
-    a.y = a0.y2;
-    a.resid = nullptr;
+    w = a0.w2;
+    y = a0.y2;
+    resid = nullptr;
     rt = rtg - a0.n_rt1;
   }
-  const uint32_t t0 = tt * kTile, r0 = rt * kTile;
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  Lane ln{lane >> 4, lane & 15, wave & 1, wave >> 1};
-  const uint32_t rows = a.w.rows, nsb = a.w.cols >> 8;
-  uint32_t rowc[2];
-#pragma unroll
-  for (int tc = 0; tc < 2; tc++) {
-    const uint32_t r = r0 + 32 * ln.rw + 16 * tc + ln.i16;
-    rowc[tc] = r < rows ? r : rows - 1;  // loads stay inside the matrix
-  }
-  float acc[2][2][4];
-#pragma unroll
-  for (int tr = 0; tr < 2; tr++)
-#pragma unroll
-    for (int tc = 0; tc < 2; tc++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) acc[tr][tc][e] = 0.0f;
+  const uint32_t t0 = tt * G::kTok, r0 = rt * G::kRows, nsb = w.cols >> 8;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  V v;
+  v.lane = threadIdx.x & 63;
+  v.l = v.lane % MT;
+  v.q = v.lane / MT;
+  v.tw = wave & 1;
+  v.rw = wave >> 1;
 
-  typename G::W wc[2], wn[2];
-  if constexpr (TY == RLH_TYPE_Q6_K) {
-    // stages by DMA (stage_dma): the copies of super-block j + 1 are issued
-    // with its weight loads and waited for before the loop's barrier
+  // Copies of half i % 2 of super-block i / 2 into a buffer of kHalfBytes.
+  // Copy n (1 KB, the tails 256 bytes) belongs to wave n % 4; every wave
+  // issues kPerWave of them (the last ones repeat copy kCopies - 1), so its
+  // vector-memory count tells which step has landed. Rows past the matrix
+  // read its last row, token tiles past the activation its last tile;
+  // neither reaches a kept output. Sources are a uniform base plus 32-bit
+  // lane offsets (32 rows' tiles at most apart).
+  const uint32_t rt_bytes = w.ntj * 64 * w.ib, rt0 = r0 / w.tr;
+  const uint8_t* wbase = w.a + (size_t)rt0 * rt_bytes;
+  const uint32_t lrow = min(r0 + v.lane % G::kRows, w.rows - 1);  // the lane's row (MT 16: rows 0..31 twice)
+  const uint32_t wlane = (lrow / w.tr - rt0) * rt_bytes + (lrow % w.tr) * 16;
+  const uint32_t tlane = (lrow / w.tr - rt0) * rt_bytes + (((lrow % w.tr) * 2) & ~3u);  // (tr is even)
+  const uint32_t last_tile = (a0.n - 1) / 32;
+  const uint8_t* xbase[2];
 #pragma unroll
-    for (int tc = 0; tc < 2; tc++) G::load(wc[tc], a.w, rowc[tc], 0, ln.q);
-    stage_dma(a, t0, 0, lds);
-    wait_vmcnt<0>();
-    __syncthreads();
-    for (uint32_t j = 0; j < nsb; j++) {
-      const bool more = j + 1 < nsb;
-      if (more) {
-        stage_dma(a, t0, j + 1, lds + ((j + 1) & 1) * kStageBytes);  // freed by the last barrier
+  for (uint32_t t = 0; t < G::kActTiles; t++)
+    xbase[t] = a0.x.p + (size_t)min(t0 / 32 + t, last_tile) * nsb * kQ8TileBytes;
+  auto copy = [&](uint32_t i, lbyte* buf) {
+    const uint32_t j = i >> 1, h = i & 1, jt = j / w.tj, jr = (j % w.tj) * w.tr;
+    const uint8_t* wt = wbase + (size_t)jt * 64 * w.ib + jr * 16;
+    const uint32_t xo = j * kQ8TileBytes;
 #pragma unroll
-        for (int tc = 0; tc < 2; tc++) G::load(wn[tc], a.w, rowc[tc], j + 1, ln.q);
-      }
-      G::compute(wc, view(lds + (j & 1) * kStageBytes), ln, acc);
-      if (more) {
-#pragma unroll
-        for (int tc = 0; tc < 2; tc++) wc[tc] = wn[tc];
-      }
-      wait_vmcnt<0>();  // this wave's copies (and weights) of super-block j + 1 have landed
-      __syncthreads();  // ... every wave's; the current buffer is free
-    }
-  } else {
-  // the Q8 bytes by DMA (stage_dma_q8), the block scales, sums and row
-  // scales through registers (they are converted or transposed on the way)
-  StageRegs sr;
-#pragma unroll
-  for (int tc = 0; tc < 2; tc++) G::load(wc[tc], a.w, rowc[tc], 0, ln.q);
-  stage_init(sr, a, t0, G::kNeedS);
-  stage_dma_q8(a, t0, 0, lds);
-  stage_load(sr, a, r0, 0, G::kNeedS, true);
-  stage_store<G::kBlockMajor>(sr, lds, G::kNeedS, true);
-  wait_vmcnt<0>();
-  __syncthreads();
-  for (uint32_t j = 0; j < nsb; j++) {
-    const bool more = j + 1 < nsb;
-    if (more) {
-      stage_dma_q8(a, t0, j + 1, lds + ((j + 1) & 1) * kStageBytes);  // freed by the last barrier
-      stage_load(sr, a, r0, j + 1, G::kNeedS, true);
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) G::load(wn[tc], a.w, rowc[tc], j + 1, ln.q);
-    }
-    G::compute(wc, view(lds + (j & 1) * kStageBytes), ln, acc);
-    if (more) {
-#pragma unroll
-      for (int tc = 0; tc < 2; tc++) wc[tc] = wn[tc];
-      stage_store<G::kBlockMajor>(sr, lds + ((j + 1) & 1) * kStageBytes, G::kNeedS, true);
-    }
-    wait_vmcnt<0>();  // this wave's copies of super-block j + 1 have landed
-    __syncthreads();  // ... every wave's; the current buffer is free
-  }
-  }
-#pragma unroll
-  for (int tr = 0; tr < 2; tr++)
-#pragma unroll
-    for (int tc = 0; tc < 2; tc++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint32_t tok = t0 + 32 * ln.tw + 16 * tr + 4 * ln.q + e;
-        const uint32_t row = r0 + 32 * ln.rw + 16 * tc + ln.i16;
-        if (tok < a.n && row < rows) {
-          const size_t idx = (size_t)tok * rows + row;
-          if (a.resid) {
-            RLH_GLOBAL float* x = (RLH_GLOBAL float*)a.resid;
-            x[idx] = x[idx] + acc[tr][tc][e];  // xs += xb (model.rs:548-552, 569-573)
-          }
-          if (a.y) ((RLH_GLOBAL float*)a.y)[idx] = acc[tr][tc][e];
+    for (uint32_t m = 0; m < G::kPerWave; m++) {
+      const uint32_t n = min(wave + 4 * m, G::kCopies - 1);
+      const uint8_t* src;
+      uint32_t off;
+      if (n < 4 * G::kActTiles) {
+        src = xbase[n >> 2] + xo + h * 4096 + (n & 3) * 1024;
+        off = v.lane * 16;
+      } else if (n < G::kActI) {
+        const uint32_t l32 = (v.lane & 31) * 16;
+        if (MT == 32) {  // scales (then sums) of both tiles
+          src = xbase[0] + xo + 8192 + (n - 8) * 1024 + h * 512;
+          off = l32 + (v.lane >= 32 ? (uint32_t)(xbase[G::kActTiles - 1] - xbase[0]) : 0u);
+        } else {  // scales and sums of the tile
+          src = xbase[0] + xo + 8192 + h * 512;
+          off = l32 + (v.lane >= 32 ? 1024u : 0u);
         }
+      } else if (n < G::kActI + G::kWI) {
+        const uint32_t p = n - G::kActI;
+        if (MT == 32) {
+          src = wt + G::chunk(p, h) * 1024;
+          off = wlane;
+        } else {  // chunks 2p and 2p + 1 of the 32 rows
+          const uint32_t c0 = G::chunk(2 * p, h), c1 = G::chunk(min(2 * p + 1, G::kCh - 1), h);
+          src = wt + c0 * 1024;
+          off = wlane + (v.lane >= 32 ? (c1 - c0) * 1024 : 0u);
+        }
+      } else {
+        src = wbase + (size_t)jt * 64 * w.ib + (w.ib / 16) * 1024 + jr * 2;
+        __builtin_amdgcn_global_load_lds((const RLH_GLOBAL void*)(src + tlane),
+                                         (RLH_LDS void*)(buf + G::kTailOff), 4, 0, 0);
+        continue;
       }
+      __builtin_amdgcn_global_load_lds((const RLH_GLOBAL void*)(src + off), (RLH_LDS void*)(buf + n * 1024), 16, 0, 0);
+    }
+  };
+
+  float acc[N];
+#pragma unroll
+  for (int e = 0; e < N; e++) acc[e] = 0.0f;
+
+  // a wave whose tokens all lie past the last one only copies
+  const bool live = t0 + MT * v.tw < a0.n;
+  const uint32_t steps = 2 * nsb / G::kHalves;
+  auto stage = [&](uint32_t i, uint32_t at) {
+#pragma unroll
+    for (uint32_t h = 0; h < G::kHalves; h++)
+      copy(i * G::kHalves + h, lds + at * G::kStageBytes + h * G::kHalfBytes);
+  };
+#pragma unroll
+  for (uint32_t s = 0; s + 1 < G::kStages; s++)
+    if (s < steps) stage(s, s);
+  uint32_t cur = 0, nxt = G::kStages - 1;  // buffers of step i and of step i + kStages - 1
+  for (uint32_t i = 0; i < steps; i++) {
+    // step i has landed: this wave's copies by its count (the later steps'
+    // copies stay in flight), the others' by the barrier, past which every
+    // wave is done with the buffer that step i + kStages - 1 takes
+    if (i + G::kStages - 2 < steps)
+      wait_vmcnt<(G::kStages - 2) * G::kHalves * G::kPerWave>();
+    else
+      wait_vmcnt<0>();
+    lds_barrier();
+    if (i + G::kStages - 1 < steps) stage(i + G::kStages - 1, nxt);
+    if (live) {
+#pragma unroll
+      for (uint32_t h = 0; h < G::kHalves; h++) {
+        v.view(lds + cur * G::kStageBytes + h * G::kHalfBytes);
+        Step<TY, MT>::run(v, G::kHalves == 1 ? i & 1 : h, acc);
+      }
+    }
+    cur = cur + 1 == G::kStages ? 0 : cur + 1;
+    nxt = nxt + 1 == G::kStages ? 0 : nxt + 1;
+  }
+  if (!live) return;  // after the last barrier
+  const uint32_t row = r0 + v.row();
+  if (row >= w.rows) return;
+  const size_t base = (size_t)(t0 + MT * v.tw + 4 * v.q) * w.rows + row;
+  const uint32_t left = a0.n - t0 - MT * v.tw;  // tokens of this wave (>= 1)
+  if (resid) {  // xs += xb (model.rs:548-552, 569-573)
+    float old[N];
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+      const uint32_t o = 8 * (e / 4) + e % 4;
+      old[e] = o + 4 * v.q < left ? ld_gf(resid + base + (size_t)o * w.rows) : 0.0f;
+    }
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+      const uint32_t o = 8 * (e / 4) + e % 4;
+      if (o + 4 * v.q < left) ((RLH_GLOBAL float*)resid)[base + (size_t)o * w.rows] = old[e] + acc[e];
+    }
+  }
+  if (y) {
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+      const uint32_t o = 8 * (e / 4) + e % 4;
+      if (o + 4 * v.q < left) ((RLH_GLOBAL float*)y)[base + (size_t)o * w.rows] = acc[e];
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -944,14 +791,51 @@ void launch_gemm_f32(hipStream_t st, const DevMat& w, const float* x, uint32_t n
   }
 }
 
-static void launch_gemm_args(hipStream_t st, uint32_t ty, const GemmArgs& a) {
+template <uint32_t TY>
+static bool set_type_lds() {
+  return hipFuncSetAttribute((const void*)k_gemm<TY, 16>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)Geo<TY, 16>::kLds) == hipSuccess &&
+         hipFuncSetAttribute((const void*)k_gemm<TY, 32>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)Geo<TY, 32>::kLds) == hipSuccess;
+}
+bool gemm_set_max_lds() {
+  return set_type_lds<RLH_TYPE_Q4_K>() && set_type_lds<RLH_TYPE_Q6_K>() && set_type_lds<RLH_TYPE_Q8_0>() &&
+         set_type_lds<RLH_TYPE_Q4_0>();
+}
+
+template <uint32_t TY, int MT>
+static void launch_variant(hipStream_t st, GemmArgs a) {
+  using G = Geo<TY, MT>;
+  a.n_tt = (a.n + G::kTok - 1) / G::kTok;
+  a.n_rt1 = (a.w.rows + G::kRows - 1) / G::kRows;
+  a.n_rt = a.n_rt1 + (a.w2.rows ? (a.w2.rows + G::kRows - 1) / G::kRows : 0);
   const uint32_t blocks = a.n_tt * ((a.n_rt + 7) / 8) * 8;
-  const size_t lds = 2 * kStageBytes;
-  switch (ty) {
-    case RLH_TYPE_Q4_K: hipLaunchKernelGGL(k_gemm<RLH_TYPE_Q4_K>, dim3(blocks), dim3(256), lds, st, a); break;
-    case RLH_TYPE_Q6_K: hipLaunchKernelGGL(k_gemm<RLH_TYPE_Q6_K>, dim3(blocks), dim3(256), lds, st, a); break;
-    case RLH_TYPE_Q8_0: hipLaunchKernelGGL(k_gemm<RLH_TYPE_Q8_0>, dim3(blocks), dim3(256), lds, st, a); break;
-    case RLH_TYPE_Q4_0: hipLaunchKernelGGL(k_gemm<RLH_TYPE_Q4_0>, dim3(blocks), dim3(256), lds, st, a); break;
+  hipLaunchKernelGGL((k_gemm<TY, MT>), dim3(blocks), dim3(256), G::kLds, st, a);
+}
+
+// 32 x 32 tiles one per wave fill the SIMDs once from 1024 tiles on; below,
+// 16 x 16 tiles make four times the waves with a quarter of the work each.
+// Both sides measured, 16 / 32: 5120 x 4096 Q4_K, 61 tokens (320 tiles) 23 /
+// 46 us; 2560 x 9728 Q6_K, 237 tokens (640) 134 / 156; 2560 x 4096 Q4_K, 237
+// tokens (640) 41 / 47; 5120 x 2560 Q4_K, 237 tokens (1280) 41 / 35; 24576 x
+// 4096 Q4_K, 61 tokens (1536) 68 / 55.
+constexpr uint64_t kTiles32 = 1024;
+
+template <uint32_t TY>
+static void launch_type(hipStream_t st, const GemmArgs& a) {
+  const uint64_t tiles = (uint64_t)((a.n + 31) / 32) * ((a.w.rows + 31) / 32 + (a.w2.rows + 31) / 32);
+  if (tiles < kTiles32)
+    launch_variant<TY, 16>(st, a);
+  else
+    launch_variant<TY, 32>(st, a);
+}
+
+static void launch_gemm_args(hipStream_t st, const GemmArgs& a) {
+  switch (a.w.ty) {
+    case RLH_TYPE_Q4_K: launch_type<RLH_TYPE_Q4_K>(st, a); break;
+    case RLH_TYPE_Q6_K: launch_type<RLH_TYPE_Q6_K>(st, a); break;
+    case RLH_TYPE_Q8_0: launch_type<RLH_TYPE_Q8_0>(st, a); break;
+    case RLH_TYPE_Q4_0: launch_type<RLH_TYPE_Q4_0>(st, a); break;
     default: break;
   }
 }
@@ -960,32 +844,26 @@ bool gemm_pair_supported(const DevMat& w, const DevMat& w2) {
   return gemm_supported(w.ty) && w2.ty == w.ty && w2.cols == w.cols;
 }
 
-void launch_gemm_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const Q8Mut& x, uint32_t n, float* y,
+void launch_gemm_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const Q8Tiles& x, uint32_t n, float* y,
                       float* y2) {
   GemmArgs a{};
   a.w = w;
   a.w2 = w2;
-  a.x = Q8Ptr{x.qs, x.d, x.s, x.s16};
+  a.x = x;
   a.n = n;
   a.y = y;
   a.y2 = y2;
-  a.n_tt = (n + kTile - 1) / kTile;
-  a.n_rt1 = (w.rows + kTile - 1) / kTile;
-  a.n_rt = a.n_rt1 + (w2.rows + kTile - 1) / kTile;
-  launch_gemm_args(st, w.ty, a);
+  launch_gemm_args(st, a);
 }
 
-void launch_gemm(hipStream_t st, const DevMat& w, const Q8Mut& x, uint32_t n, float* y, float* resid) {
+void launch_gemm(hipStream_t st, const DevMat& w, const Q8Tiles& x, uint32_t n, float* y, float* resid) {
   GemmArgs a{};
   a.w = w;
-  a.x = Q8Ptr{x.qs, x.d, x.s, x.s16};
+  a.x = x;
   a.n = n;
   a.y = y;
   a.resid = resid;
-  a.n_tt = (n + kTile - 1) / kTile;
-  a.n_rt = (w.rows + kTile - 1) / kTile;
-  a.n_rt1 = a.n_rt;
-  launch_gemm_args(st, w.ty, a);
+  launch_gemm_args(st, a);
 }
 
 }  // namespace rlh

@@ -18,6 +18,12 @@ void launch_embed(hipStream_t st, const DevMat& w, const uint32_t* tok, uint32_t
 void launch_rmsnorm_q8(hipStream_t st, const float* x, const float* w, uint32_t n, uint32_t n_tok, float eps,
                        const Q8Buf& out, float* xb);
 void launch_quantize_q8(hipStream_t st, const float* x, uint32_t n, const Q8Buf& out);
+// The tiled forms of a prefill batch (n_tok tokens).
+void launch_rmsnorm_q8(hipStream_t st, const float* x, const float* w, uint32_t n, uint32_t n_tok, float eps,
+                       const Q8Tiles& out, float* xb);
+void launch_quantize_q8(hipStream_t st, const float* x, uint32_t n_tok, const Q8Tiles& out);
+void launch_swiglu_q8(hipStream_t st, const float* g, const float* u, uint32_t n_tok, const Q8Tiles& out,
+                      float* h_out);
 void launch_block_dots(hipStream_t st, const DevMat& w, const int8_t* a, int32_t* out, uint32_t per_row);
 void launch_dequant(hipStream_t st, const DevMat& w, float* out);
 void launch_qk_norm_rope_kv(hipStream_t st, float* q, float* k, const float* v, const float* bq, const float* bk,

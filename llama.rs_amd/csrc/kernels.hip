@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "kernels.h"
 #include "rlh_device.h"
 
@@ -28,7 +30,9 @@ __global__ void __launch_bounds__(256) k_embed(DevMat w, const uint32_t* tok, fl
 // result: xb = (x*s)*w, s = 1/sqrt(ss/n + eps); Q8 blocks of xb.
 // One 256-thread block per token (grid.x = n_tokens). n % 32 == 0.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_rmsnorm_q8(const float* x, const float* w, int n, float eps, Q8Out out,
+// OUT: Q8Out (rows) or Q8Tiles (the batch layout of the prefill products).
+template <class OUT>
+__global__ void __launch_bounds__(256) k_rmsnorm_q8(const float* x, const float* w, int n, float eps, OUT out,
                                                     float* xb) {
   __shared__ float s_scale;
   __shared__ __attribute__((aligned(16))) float xs_generic[kMaxEmbd];
@@ -64,9 +68,6 @@ __global__ void __launch_bounds__(256) k_rmsnorm_q8(const float* x, const float*
   }
   __syncthreads();
   const float s = s_scale;
-  const uint32_t nb = (uint32_t)n / 32;
-  Q8Out o{out.qs + (size_t)blockIdx.x * n, out.d + (size_t)blockIdx.x * nb, out.s + (size_t)blockIdx.x * nb,
-          out.s16 + (size_t)blockIdx.x * nb * 2};
   // xb = (x * s) * w; 8 consecutive threads hold one Q8 block (4 values each).
 #pragma unroll
   for (int k = 0; k < kV; k++) {
@@ -81,9 +82,18 @@ __global__ void __launch_bounds__(256) k_rmsnorm_q8(const float* x, const float*
         xo[2] = v2;
         xo[3] = v3;
       }
-      q8_quant_block8x4(v0, v1, v2, v3, o, (uint32_t)i / 8);
+      if constexpr (std::is_same<OUT, Q8Tiles>::value)
+        q8_quant_block8x4(v0, v1, v2, v3, out, blockIdx.x, (uint32_t)i / 8);
+      else
+        q8_quant_block8x4(v0, v1, v2, v3, out, blockIdx.x * ((uint32_t)n / 32) + (uint32_t)i / 8);
     }
   }
+}
+
+// quantize_q8 of every token of a batch into tiles: grid (cols / 256, n).
+__global__ void __launch_bounds__(256) k_quantize_q8_tiles(const float* x, Q8Tiles out) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x, tok = blockIdx.y;
+  q8_quant_block32(x[(size_t)tok * out.nsb * 256 + i], out, tok, i / 32);
 }
 
 // Standalone quantize_q8 (op-level entry): grid covers n/32 blocks, 8 per block.
@@ -247,6 +257,28 @@ __global__ void __launch_bounds__(256) k_swiglu_q8(const float* g, const float* 
   q8_quant_block8x4(h0, h1, h2, h3, out, i4 / 8);
 }
 
+// The same for a batch's tiles: grid (F / 32, ceil(n / 32)), a block per 32
+// tokens of one Q8 block column, eight threads per token (each token's 32
+// gate and up values are one 128-byte line; the block's quants fill the
+// tile's 1 KB of that column).
+__global__ void __launch_bounds__(256) k_swiglu_q8_tiles(const float* g, const float* u, uint32_t n, Q8Tiles out,
+                                                         float* h_out) {
+  __shared__ uint64_t tab_g[32];
+  lu64* tab = (lu64*)tab_g;
+  exp_tab_to_lds(tab);
+  __syncthreads();
+  const uint32_t tok = blockIdx.y * 32 + threadIdx.x / 8, F = out.nsb * 256;
+  if (tok >= n) return;  // whole groups of eight threads
+  const size_t i4 = (size_t)tok * (F / 4) + blockIdx.x * 8 + (threadIdx.x & 7);
+  const float4 x = ((const float4*)g)[i4], uu = ((const float4*)u)[i4];
+  const float h0 = (x.x / (1.0f + expf_glibc_t(-x.x, tab))) * uu.x;
+  const float h1 = (x.y / (1.0f + expf_glibc_t(-x.y, tab))) * uu.y;
+  const float h2 = (x.z / (1.0f + expf_glibc_t(-x.z, tab))) * uu.z;
+  const float h3 = (x.w / (1.0f + expf_glibc_t(-x.w, tab))) * uu.w;
+  if (h_out) ((float4*)h_out)[i4] = float4{h0, h1, h2, h3};
+  q8_quant_block8x4(h0, h1, h2, h3, out, tok, blockIdx.x);
+}
+
 // ---------------------------------------------------------------------------
 // Argmax with main.rs:453-463 semantics: start at -inf, strict '>' so the
 // lowest index among equal maxima wins and NaN never wins.
@@ -351,7 +383,25 @@ void launch_embed(hipStream_t st, const DevMat& w, const uint32_t* tok, uint32_t
 
 void launch_rmsnorm_q8(hipStream_t st, const float* x, const float* w, uint32_t n, uint32_t n_tok, float eps,
                        const Q8Buf& out, float* xb) {
-  hipLaunchKernelGGL(k_rmsnorm_q8, dim3(n_tok), dim3(256), 0, st, x, w, (int)n, eps, q8out(out), xb);
+  hipLaunchKernelGGL(k_rmsnorm_q8<Q8Out>, dim3(n_tok), dim3(256), 0, st, x, w, (int)n, eps, q8out(out), xb);
+}
+void launch_rmsnorm_q8(hipStream_t st, const float* x, const float* w, uint32_t n, uint32_t n_tok, float eps,
+                       const Q8Tiles& out, float* xb) {
+  hipLaunchKernelGGL(k_rmsnorm_q8<Q8Tiles>, dim3(n_tok), dim3(256), 0, st, x, w, (int)n, eps, out, xb);
+}
+void launch_quantize_q8(hipStream_t st, const float* x, uint32_t n_tok, const Q8Tiles& out) {
+  // the grid's y dimension holds 65535 rows: longer batches go in parts of whole tiles
+  constexpr uint32_t kMost = 65504;
+  for (uint32_t t = 0; t < n_tok; t += kMost) {
+    const Q8Tiles o{out.p + (size_t)(t / 32) * out.nsb * kQ8TileBytes, out.nsb};
+    hipLaunchKernelGGL(k_quantize_q8_tiles, dim3(out.nsb, n_tok - t < kMost ? n_tok - t : kMost), dim3(256), 0, st,
+                       x + (size_t)t * out.nsb * 256, o);
+  }
+}
+void launch_swiglu_q8(hipStream_t st, const float* g, const float* u, uint32_t n_tok, const Q8Tiles& out,
+                      float* h_out) {
+  hipLaunchKernelGGL(k_swiglu_q8_tiles, dim3(out.nsb * 8, (n_tok + 31) / 32), dim3(256), 0, st, g, u, n_tok, out,
+                     h_out);
 }
 
 void launch_quantize_q8(hipStream_t st, const float* x, uint32_t n, const Q8Buf& out) {

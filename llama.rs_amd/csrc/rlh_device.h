@@ -278,6 +278,26 @@ __device__ __forceinline__ void q8_quant_block32(float v, Q8Out o, uint32_t blk)
   }
 }
 
+// The same as block blk of token tok of a tiled batch (rlh_format.h).
+__device__ __forceinline__ void q8_quant_block32(float v, const Q8Tiles& o, uint32_t tok, uint32_t blk) {
+  const uint32_t l = threadIdx.x & 31, kb = blk & 7, t = tok & 31;
+  float a = fabsf(v);
+#pragma unroll
+  for (int m = 16; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, 32));
+  const float d = a / 127.0f;
+  const float inv = d > 0.0f ? 1.0f / d : 0.0f;
+  const int q = cvtps_packs_i8(__builtin_rintf(v * inv));
+  int s = q;
+#pragma unroll
+  for (int m = 16; m >= 1; m >>= 1) s += __shfl_xor(s, m, 32);
+  RLH_GLOBAL uint8_t* b = (RLH_GLOBAL uint8_t*)o.p + ((size_t)(tok >> 5) * o.nsb + (blk >> 3)) * kQ8TileBytes;
+  b[kb * 1024 + (l >> 3 & 1) * 512 + t * 16 + (l >> 4) * 8 + (l & 7)] = (uint8_t)q;
+  if (l == 0) {
+    *(RLH_GLOBAL float*)(b + 8192 + kb * 128 + t * 4) = d;
+    *(RLH_GLOBAL int32_t*)(b + 9216 + kb * 128 + t * 4) = s;
+  }
+}
+
 // The same for a whole wave holding two blocks, lanes 0..31 = block blk and
 // 32..63 = block blk + 1 (every lane active; the stores of half h happen
 // when store[h]). The reductions use DPP instead of LDS-routed shuffles:
@@ -385,6 +405,17 @@ __device__ __forceinline__ void q8_quant_block8x4(float v0, float v1, float v2, 
   } else if (l == 4) {
     ((RLH_GLOBAL int32_t*)o.s16)[(size_t)blk * 2 + 1] = r.s;
   }
+}
+
+// The same block as block blk of token tok of a tiled batch (rlh_format.h).
+__device__ __forceinline__ void q8_quant_block8x4(float v0, float v1, float v2, float v3, const Q8Tiles& o,
+                                                  uint32_t tok, uint32_t blk) {
+  const uint32_t l = threadIdx.x & 7, kb = blk & 7, t = tok & 31;
+  const Q8Blk8x4 r = q8_block8x4(v0, v1, v2, v3);
+  RLH_GLOBAL uint8_t* b = (RLH_GLOBAL uint8_t*)o.p + ((size_t)(tok >> 5) * o.nsb + (blk >> 3)) * kQ8TileBytes;
+  *(RLH_GLOBAL uint32_t*)(b + kb * 1024 + (l >> 1 & 1) * 512 + t * 16 + (l >> 2) * 8 + (l & 1) * 4) = r.packed;
+  if (l == 0) *(RLH_GLOBAL float*)(b + 8192 + kb * 128 + t * 4) = r.d;
+  if (l == 4) *(RLH_GLOBAL int32_t*)(b + 9216 + kb * 128 + t * 4) = r.tot;
 }
 
 // Sum of squares of rmsnorm_core (simd.rs:285-313) over a row staged in LDS,

@@ -79,4 +79,21 @@ struct Q8Mut {
   int32_t* s16;
 };
 
+// Q8 activation rows of a batch (prefill), in tiles of 32 tokens x 256 values
+// laid out as the MFMA operands take them. Tile (T, j) of a batch with
+// cols / 256 = nsb super-blocks starts at (T * nsb + j) * kQ8TileBytes:
+//   qs   8 blocks x 1 KB: value p of block kb of token t at
+//        kb * 1024 + (p / 8 % 2) * 512 + t * 16 + (p / 16) * 8 + p % 8
+//   d    f32 [8 blocks][32 tokens] at 8192
+//   s    i32 [8 blocks][32 tokens] at 9216 (the block sums)
+// so a tile is copied into LDS as it lies and one 16-byte (8-byte) read per
+// lane is an operand of a 32 x 32 (16 x 16) MFMA. The last tile's tokens past
+// the batch hold nothing.
+constexpr uint32_t kQ8TileBytes = 10240;
+struct Q8Tiles {
+  uint8_t* p;
+  uint32_t nsb;
+};
+inline uint64_t q8_tiles_bytes(uint64_t n, uint64_t cols) { return (n + 31) / 32 * (cols / 256) * kQ8TileBytes; }
+
 }  // namespace rlh

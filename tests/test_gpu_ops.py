@@ -158,3 +158,48 @@ def test_matvec_rejects_bad_shape():
     with pytest.raises(rlh.RlhError) as e:
         rlh.matvec(Q4_K, w, 1, 100, np.zeros(100, np.float32))
     assert e.value.code == rlh.RLH_EINVAL
+
+
+# matmul_batch's integer products at the edges of their tiles: 16 x 16 wave
+# tiles (fewer than 1024 tiles of 32 x 32) with token counts around 16 and
+# 32, rows around 32, one to five super-blocks (four are staged at a time);
+# 32 x 32 wave tiles (2080 rows x 527 tokens: 65 x 17 = 1105 tiles) with a
+# last tile of rows and of tokens partly or wholly empty.
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("rows,cols,n", [(1, 256, 2), (33, 256, 16), (31, 512, 17), (65, 768, 33), (96, 1024, 31),
+                                         (40, 1280, 64), (2080, 256, 527), (2049, 768, 513), (2200, 512, 480)])
+def test_matmul_batch_tiles_bit_exact(ty, rows, cols, n):
+    print(f"matmul_batch ty={ty} {rows}x{cols} n={n}", flush=True)
+    rng = np.random.default_rng(rows + cols + n + ty)
+    bs, ts = BLOCK[ty]
+    w = random_blocks(ty, rows * cols // bs, rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    got = rlh.matmul_batch(ty, w, rows, cols, x, n)
+    ref = oracle.matmul_batch(ty, w, rows, cols, x, n, oracle.MODE_BATCH_INT)
+    assert np.array_equal(bits(got), bits(ref))
+
+
+@pytest.mark.parametrize("ty", TYPES)
+@pytest.mark.parametrize("rows,n", [(40, 37), (2100, 500)])
+def test_matmul_batch_special_scales(ty, rows, n):
+    """f16 scales that are infinite, NaN, zero, subnormal, the largest finite
+    one and negative (the products take them times a power of two)."""
+    print(f"matmul_batch special scales ty={ty} {rows} n={n}", flush=True)
+    rng = np.random.default_rng(7 * ty + rows)
+    bs, ts = BLOCK[ty]
+    cols = 512
+    raw = random_blocks(ty, rows * cols // bs, rng).reshape(-1, ts)
+    at = {Q4_K: [0, 2], Q6_K: [208]}.get(ty, [0])
+    for col in at:
+        for bits16 in (0x7C00, 0xFC00, 0x7E00, 0x0000, 0x8000, 0x0001, 0x03FF, 0x7BFF, 0xC000):
+            hit = rng.integers(0, len(raw), max(1, len(raw) // 100))
+            raw[hit, col], raw[hit, col + 1] = bits16 & 0xFF, bits16 >> 8
+    w = raw.reshape(-1)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[::5, 32:64] = 0.0  # zero blocks: zero dots against every scale
+    got = np.asarray(rlh.matmul_batch(ty, w, rows, cols, x, n))
+    with np.errstate(all="ignore"):
+        ref = np.asarray(oracle.matmul_batch(ty, w, rows, cols, x, n, oracle.MODE_BATCH_INT))
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint32), ref[~nan].view(np.uint32))
