@@ -1039,6 +1039,16 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
       else
         launch_gemm_f32(s, w, xf, mtok, n4, y, resid);
     };
+    auto pair_supported = [](const DevMat& w, const DevMat& w2) {
+      return gemm_pair_supported(w, w2) || gemm_f32_pair_supported(w, w2);
+    };
+    auto pair_on = [&](hipStream_t s, const DevMat& w, const DevMat& w2, const Q8Tiles& q8, const float* xf, float* y,
+                       float* y2) {
+      if (gemm_supported(w.ty))
+        launch_gemm_pair(s, w, w2, q8, mtok, y, y2);
+      else
+        launch_gemm_f32_pair(s, w, w2, xf, mtok, n4, y, y2);
+    };
     auto product = [&](const DevMat& w, const Q8Tiles& q8, const float* xf, float* y, float* resid) {
       product_on(st, w, q8, xf, y, resid);
     };
@@ -1055,10 +1065,10 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
       bool v_pending = false;  // the main stream has yet to wait for the v stream
       // q and k of one type and width: one launch of both (no stream join
       // for k on the way to the next kernel)
-      const bool qk_pair = gemm_pair_supported(L.q.dm, L.k.dm);
+      const bool qk_pair = pair_supported(L.q.dm, L.k.dm);
       auto q_and_k = [&](hipStream_t s) {
         if (qk_pair) {
-          launch_gemm_pair(s, L.q.dm, L.k.dm, c->act_eb, mtok, c->qb, c->kb);
+          pair_on(s, L.q.dm, L.k.dm, c->act_eb, xn, c->qb, c->kb);
         } else {
           product_on(s, L.q.dm, c->act_eb, xn, c->qb, nullptr);
           product_on(s, L.k.dm, c->act_eb, xn, c->kb, nullptr);
@@ -1119,8 +1129,8 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
       launch_attn_pv(st, a, false);
       product(L.o.dm, c->act_qb, c->attnb, nullptr, c->xb);
       launch_rmsnorm_q8(st, c->xb, L.ffn_norm.p, E, mtok, eps, c->act_eb, xn);
-      if (gemm_pair_supported(L.gate.dm, L.up.dm)) {  // one launch of both (one boundary less)
-        launch_gemm_pair(st, L.gate.dm, L.up.dm, c->act_eb, mtok, c->gb, c->ub);
+      if (pair_supported(L.gate.dm, L.up.dm)) {  // one launch of both (one boundary less)
+        pair_on(st, L.gate.dm, L.up.dm, c->act_eb, xn, c->gb, c->ub);
       } else {
         product(L.gate.dm, c->act_eb, xn, c->gb, nullptr);
         product(L.up.dm, c->act_eb, xn, c->ub, nullptr);

@@ -41,5 +41,9 @@ void launch_gemm_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const Q
 bool gemm_f32_supported(uint32_t ty);
 void launch_gemm_f32(hipStream_t st, const DevMat& w, const float* x, uint32_t n, uint32_t n4, float* y,
                      float* resid);
+// Two of them with one activation in one launch (same type and columns).
+bool gemm_f32_pair_supported(const DevMat& w, const DevMat& w2);
+void launch_gemm_f32_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const float* x, uint32_t n, uint32_t n4,
+                          float* y, float* y2);
 
 }  // namespace rlh

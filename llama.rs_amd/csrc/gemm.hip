@@ -549,19 +549,40 @@ __global__ void __launch_bounds__(256, 4) k_gemm(GemmArgs a0) {
 // (32 chains over 32-value chunks, (a0+a1)+(a2+a3), tree). ys starts at zero
 // and gets `+= value`. F32 weights take matmul_batch's F32 fast path
 // (ops.rs:165-174): dot(row, x) for every token, stored as is.
-// Block: 16 rows x 16 tokens, one thread per (row, token) running its
-// chains; each 256-value super-block of the 16 rows is dequantized into LDS
-// once and the 16 tokens' activations staged beside it.
+//
+// The chains run on the f32 MFMA, whose result is the chain of fused
+// multiply-adds over k = 0, 1, .. in order, rounded at each (every depth and
+// shape; subnormals, infinities and NaN as fmaf), at twice the rate of
+// v_fma_f32. A 16 x 16 x 4 product of tokens x rows over elements 32 p + 8 k
+// + l (k = 0..3) is four steps of chain l of dot_multi_rows. The same
+// weight operand in sixteen 4 x 4 x 1 blocks (4 single tokens; block 4 k + g
+// = rows 4 g .. + 3) is one step of the chains (k, l) of dot_f32_avx2. A
+// lane's operands of all eight l are 32 consecutive bytes.
+//
+// Block: 16 RT rows x up to 4 jobs, one wave per job; a job is 16 tokens in
+// groups of four, or 4 single tokens (32 RT accumulators either way). 256 /
+// RT values of the rows (16 per thread) are dequantized into the second of
+// two LDS buffers while the current ones are multiplied; the activations
+// come straight from memory (each token's 32 values of a step are one
+// 128-byte line), two steps ahead. A 9728 x 2560 Q5_K pair with 131 tokens:
+// 658 us with one FMA chain per thread, 191 us; its multiply-adds alone take
+// 83 us at the f32 MFMA rate, which no VALU work overlaps (the dequantizing
+// adds to it).
 // ---------------------------------------------------------------------------
-constexpr uint32_t kFR = 16, kFT = 16, kFS = 260;  // rows, tokens, LDS floats per 256 values
+constexpr uint32_t kFT = 16;  // tokens per grouped job
 
 struct GemmF32Args {
   DevMat w;
+  DevMat w2;       // a second segment of the same type and columns (rows 0: none)
   const float* x;  // [n][cols] f32
   uint32_t n;
   float* y;
-  float* resid;
+  float* y2;
+  float* resid;    // of the first segment
   uint32_t n4;     // tokens handled in groups of 4 (n - n % 4)
+  uint32_t n_jb;   // blocks per row tile: jobs / 4, rounded up
+  uint32_t n_rt;   // row tiles of both segments
+  uint32_t n_rt1;  // row tiles of w
 };
 
 __device__ __forceinline__ float tree8(const float* A) {
@@ -605,12 +626,10 @@ struct Dq16 {
       const uint32_t dsub = dp / 2;
       const u32x4_t hdr = v[0], qv = v[1], hv = v[2];
       const float d = f16_to_f32(hdr.x & 0xffff), dmin = f16_to_f32(hdr.x >> 16);
-      uint8_t sb[12];
-      const uint32_t sw[3] = {hdr.y, hdr.z, hdr.w};
-#pragma unroll
-      for (int k = 0; k < 12; k++) sb[k] = (uint8_t)(sw[k / 4] >> (8 * (k % 4)));
-      uint32_t sc, m;
-      scale_min_k4((int)dsub, sb, sc, m);
+      // get_scale_min_k4 (quant.rs:176-185)
+      const uint32_t sh = 8 * (dsub & 3), s0 = hdr.y >> sh, s1 = hdr.z >> sh, s2 = hdr.w >> sh;
+      const uint32_t sc = dsub < 4 ? s0 & 63 : (s2 & 15) | (s0 >> 2 & 48);
+      const uint32_t m = dsub < 4 ? s1 & 63 : (s2 >> 4 & 15) | (s1 >> 2 & 48);
       const float d1 = d * (float)sc, mm1 = dmin * (float)m;
       const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w}, hw[4] = {hv.x, hv.y, hv.z, hv.w};
 #pragma unroll
@@ -664,97 +683,143 @@ struct Dq16 {
   }
 };
 
-template <uint32_t TY>
-__global__ void __launch_bounds__(256) k_gemm_f32(GemmF32Args a) {
-  __shared__ __attribute__((aligned(16))) float ws_g[kFR * kFS];
-  __shared__ __attribute__((aligned(16))) float xs_g[kFT * kFS];
+template <uint32_t TY, int RT>
+__global__ void __launch_bounds__(256, 3) k_gemm_f32(GemmF32Args a) {
+  constexpr uint32_t kFR = 16 * RT, kFV = 256 / RT, kFS = kFV + 4;  // rows, values per stage, LDS row stride
+  __shared__ __attribute__((aligned(16))) float ws_g[2][kFR * kFS];
   typedef RLH_LDS float lfloat;
   typedef RLH_LDS f32x4_t lf32x4;
   lfloat* ws = (lfloat*)ws_g;
-  lfloat* xs = (lfloat*)xs_g;
-  const uint32_t tid = threadIdx.x, r0 = blockIdx.x * kFR, t0 = blockIdx.y * kFT;
-  const uint32_t rl = tid / kFT, tl = tid % kFT, row = r0 + rl, tok = t0 + tl;
-  const uint32_t nsb = a.w.cols / 256;
-  const bool tail = tok >= a.n4;
-  // dequant duty: row r0 + tid / 16, values 16 * (tid % 16) .. + 15 of the super-block
-  const uint32_t dr = tid / 16, dp = tid % 16;
-  const uint32_t drow = min(r0 + dr, a.w.rows - 1);
-  float c8[8], c32[4][8];
-#pragma unroll
-  for (int l = 0; l < 8; l++) {
-    c8[l] = 0.0f;
-#pragma unroll
-    for (int m = 0; m < 4; m++) c32[m][l] = 0.0f;
+  // XCD-aware order as in k_gemm
+  const uint32_t b = blockIdx.x, k = b >> 3;
+  const uint32_t jb = k % a.n_jb, rtg = (k / a.n_jb) * 8 + (b & 7);
+  if (rtg >= a.n_rt) return;  // whole block, before any barrier
+  DevMat w = a.w;
+  float *y = a.y, *resid = a.resid;
+  uint32_t r0 = rtg * kFR;
+  if (rtg >= a.n_rt1) {
+    w = a.w2;
+    y = a.y2;
+    resid = nullptr;
+    r0 = (rtg - a.n_rt1) * kFR;
   }
-  for (uint32_t j = 0; j < nsb; j++) {
-    Dq16<TY> dq;
-    dq.load(a.w, drow, j, dp);
-    f32x4_t xv[4];
-    const uint32_t xt = min(t0 + tid / 16, a.n - 1);
+  const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t l = tid & 15, q = (tid >> 4) & 3;
+  const uint32_t S = w.cols / 32, nh = w.cols / kFV;
+  // the wave's job: the jobs spread evenly over the row tile's blocks, the
+  // slots without one over the waves (each wave has a SIMD of its own)
+  const uint32_t nm = (a.n4 + kFT - 1) / kFT, jobs = nm + (a.n - a.n4 + 3) / 4;
+  const uint32_t per = (jobs + a.n_jb - 1) / a.n_jb, slot = (wave + b / 8 + rtg) & 3, job = per * jb + slot;
+  const bool live = slot < per && job < jobs, single = job >= nm;
+  const uint32_t tok0 = single ? a.n4 + (job - nm) * 4 : job * kFT, tok_end = single ? a.n : a.n4;
+  const float* xp = a.x + (size_t)(live ? min(tok0 + (single ? l & 3 : l), tok_end - 1) : 0u) * w.cols + 8 * q;
+  f32x4_t xv[4][2];  // steps p .. p + 2
+  auto load_x = [&](uint32_t p) {
+    const float* src = xp + 32 * min(p, S - 1);
+    xv[p & 3][0] = *(const RLH_GLOBAL f32x4_t*)src;
+    xv[p & 3][1] = *(const RLH_GLOBAL f32x4_t*)(src + 4);
+  };
+  // dequant duty: 16 values (piece dpc) of one of the block's rows
+  constexpr uint32_t kPc = kFV / 16;
+  const uint32_t drow = min(r0 + tid / kPc, w.rows - 1), dpc = tid % kPc;
+  Dq16<TY> dq;
+  auto load_w = [&](uint32_t h) { dq.load(w, drow, h / RT, kPc * (h % RT) + dpc); };
+  auto store_w = [&](uint32_t h) {
+    lfloat* o = ws + (h & 1) * (kFR * kFS) + (tid / kPc) * kFS + 16 * dpc;
+    f32x4_t v[4];
+    dq.values(kPc * (h % RT) + dpc, v);
 #pragma unroll
-    for (int q = 0; q < 4; q++)  // token t0 + tid / 16, values 16 * (tid % 16) + 4q
-      xv[q] = *(const RLH_GLOBAL f32x4_t*)(a.x + (size_t)xt * a.w.cols + 256 * j + 16 * (tid % 16) + 4 * q);
-    f32x4_t wv[4];
-    dq.values(dp, wv);
-    __syncthreads();  // the previous super-block's tiles are consumed
+    for (int i = 0; i < 4; i++) *(lf32x4*)(o + 4 * i) = v[i];
+  };
+  auto el = [](const f32x4_t (&v)[2], int c) { return v[c >> 2][c & 3]; };
+
+  load_w(0);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      *(lf32x4*)(ws + dr * kFS + 16 * dp + 4 * q) = wv[q];
-      *(lf32x4*)(xs + (tid / 16) * kFS + 16 * (tid % 16) + 4 * q) = xv[q];
+  for (uint32_t p = 0; p < 2; p++) load_x(p);
+  store_w(0);
+  if (nh > 1) load_w(1);
+  lds_barrier();
+  // one loop per kind of job (a condition inside one loop would make the
+  // compiler copy the accumulators); all meet the same barriers
+  auto sweep = [&](auto mul) {
+    for (uint32_t h = 0; h < nh; h++) {
+      if (h + 1 < nh) store_w(h + 1);  // that buffer's last readers passed the barrier that ended h - 1
+      if (h + 2 < nh) load_w(h + 2);
+      const lfloat* wb = ws + (h & 1) * (kFR * kFS) + l * kFS + 8 * q;
+      mul(h, wb);
+      lds_barrier();
     }
-    __syncthreads();
-    const lf32x4* w4 = (const lf32x4*)(ws + rl * kFS);
-    const lf32x4* x4 = (const lf32x4*)(xs + tl * kFS);
-    if (!tail) {  // dot_multi_rows: lane l of the 8-wide chain takes 8i + l
-#pragma unroll 8
-      for (int i = 0; i < 32; i++) {
-        const f32x4_t wa = w4[2 * i], wb = w4[2 * i + 1], xa = x4[2 * i], xb = x4[2 * i + 1];
-        c8[0] = __builtin_fmaf(wa.x, xa.x, c8[0]);
-        c8[1] = __builtin_fmaf(wa.y, xa.y, c8[1]);
-        c8[2] = __builtin_fmaf(wa.z, xa.z, c8[2]);
-        c8[3] = __builtin_fmaf(wa.w, xa.w, c8[3]);
-        c8[4] = __builtin_fmaf(wb.x, xb.x, c8[4]);
-        c8[5] = __builtin_fmaf(wb.y, xb.y, c8[5]);
-        c8[6] = __builtin_fmaf(wb.z, xb.z, c8[6]);
-        c8[7] = __builtin_fmaf(wb.w, xb.w, c8[7]);
-      }
-    } else {  // dot_f32_avx2: chain (m, l) takes 32c + 8m + l
-#pragma unroll 2
-      for (int c = 0; c < 8; c++) {
+  };
+  auto products = [&](auto step) {
+    sweep([&](uint32_t h, const lfloat* wb) {
+      f32x4_t wv[2][2];  // of product i (step i / RT, rows 16 (i % RT) ..) and of the next one
+      auto read_w = [&](int i) {
+        const lfloat* wp = wb + 16 * (i % RT) * kFS + 32 * (i / RT);
+        wv[i & 1][0] = *(const lf32x4*)wp;
+        wv[i & 1][1] = *(const lf32x4*)(wp + 4);
+      };
+      read_w(0);
 #pragma unroll
-        for (int mq = 0; mq < 4; mq++) {
-          const f32x4_t wa = w4[8 * c + 2 * mq], wb = w4[8 * c + 2 * mq + 1];
-          const f32x4_t xa = x4[8 * c + 2 * mq], xb = x4[8 * c + 2 * mq + 1];
-          c32[mq][0] = __builtin_fmaf(wa.x, xa.x, c32[mq][0]);
-          c32[mq][1] = __builtin_fmaf(wa.y, xa.y, c32[mq][1]);
-          c32[mq][2] = __builtin_fmaf(wa.z, xa.z, c32[mq][2]);
-          c32[mq][3] = __builtin_fmaf(wa.w, xa.w, c32[mq][3]);
-          c32[mq][4] = __builtin_fmaf(wb.x, xb.x, c32[mq][4]);
-          c32[mq][5] = __builtin_fmaf(wb.y, xb.y, c32[mq][5]);
-          c32[mq][6] = __builtin_fmaf(wb.z, xb.z, c32[mq][6]);
-          c32[mq][7] = __builtin_fmaf(wb.w, xb.w, c32[mq][7]);
+      for (int i = 0; i < 8; i++) {
+        if (i % RT == 0) load_x(kFV / 32 * h + i / RT + 2);
+        if (i < 7) read_w(i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 8; c++) step(i % RT, c, el(xv[(i / RT) & 3], c), el(wv[i & 1], c));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+  };
+  auto put = [&](uint32_t tok, uint32_t row, float v) {
+    if (tok >= tok_end || row >= w.rows) return;
+    const size_t idx = (size_t)tok * w.rows + row;
+    if (resid) {
+      RLH_GLOBAL float* o = (RLH_GLOBAL float*)resid;
+      o[idx] = o[idx] + v;
+    }
+    if (y) ((RLH_GLOBAL float*)y)[idx] = v;
+  };
+  f32x4_t acc[RT][8];
+#pragma unroll
+  for (int t = 0; t < RT; t++)
+#pragma unroll
+    for (int c = 0; c < 8; c++) acc[t][c] = f32x4_t{};
+  if (!live) {
+    sweep([](uint32_t, const lfloat*) {});
+  } else if (!single) {  // element e of a lane: token 4 q + e, row l
+    products([&](int t, int c, float xe, float we) {
+      acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(xe, we, acc[t][c], 0, 0, 0);
+    });
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float c8[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) c8[c] = acc[t][c][e];
+        // out += hsum(acc) + tail (no tail: cols % 8 == 0)
+        put(tok0 + 4 * q + e, r0 + 16 * t + l, 0.0f + (tree8(c8) + 0.0f));
+      }
+  } else {  // element e of a lane: token e, row l, chains (q, c)
+    products([&](int t, int c, float xe, float we) {
+      acc[t][c] = __builtin_amdgcn_mfma_f32_4x4x1f32(xe, we, acc[t][c], 0, 0, 0);
+    });
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float A[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) {  // (a0 + a1) + (a2 + a3) over the lane groups
+          const float s = acc[t][c][e] + __shfl_xor(acc[t][c][e], 16);
+          A[c] = s + __shfl_xor(s, 32);
         }
+        // F32 weights store dot(row, x) (ops.rs:169-173); the others add it to
+        // the zeroed output (ops.rs:236 ys.fill, then +=)
+        const float v = TY == RLH_TYPE_F32 ? tree8(A) : 0.0f + tree8(A);
+        if (q == 0) put(tok0 + e, r0 + 16 * t + l, v);
       }
-    }
   }
-  if (row >= a.w.rows || tok >= a.n) return;
-  float v;
-  if (!tail) {
-    v = 0.0f + (tree8(c8) + 0.0f);  // out += hsum(acc) + tail (no tail: cols % 8 == 0)
-  } else {
-    float A[8];
-#pragma unroll
-    for (int l = 0; l < 8; l++) A[l] = (c32[0][l] + c32[1][l]) + (c32[2][l] + c32[3][l]);
-    // F32 weights store dot(row, x) (ops.rs:169-173); the others add it to
-    // the zeroed output (ops.rs:236 ys.fill, then +=)
-    v = TY == RLH_TYPE_F32 ? tree8(A) : 0.0f + tree8(A);
-  }
-  const size_t idx = (size_t)tok * a.w.rows + row;
-  if (a.resid) {
-    RLH_GLOBAL float* x = (RLH_GLOBAL float*)a.resid;
-    x[idx] = x[idx] + v;
-  }
-  if (a.y) ((RLH_GLOBAL float*)a.y)[idx] = v;
 }
 
 }  // namespace
@@ -768,6 +833,38 @@ bool gemm_f32_supported(uint32_t ty) {
          ty == RLH_TYPE_F16 || ty == RLH_TYPE_BF16 || ty == RLH_TYPE_F32;
 }
 
+template <uint32_t TY>
+static void launch_f32_type(hipStream_t st, GemmF32Args a) {
+  const uint32_t jobs = (a.n4 + kFT - 1) / kFT + (a.n - a.n4 + 3) / 4;
+  a.n_jb = (jobs + 3) / 4;
+  // 32-row blocks unless they are too few to give every CU two: 2560 x 4096
+  // Q5_K with 131 tokens (240 blocks of 32 rows) 52 / 56 us with 16 / 32
+  // rows, 19456 x 2560 with 20 (1216) 67 / 61
+  const uint64_t blocks32 = (uint64_t)a.n_jb * ((a.w.rows + 31) / 32 + (a.w2.rows + 31) / 32);
+  const uint32_t fr = blocks32 < 512 ? 16 : 32;
+  a.n_rt1 = (a.w.rows + fr - 1) / fr;
+  a.n_rt = a.n_rt1 + (a.w2.rows + fr - 1) / fr;
+  const dim3 grid(a.n_jb * ((a.n_rt + 7) / 8) * 8);
+  if (fr == 16)
+    hipLaunchKernelGGL((k_gemm_f32<TY, 1>), grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_gemm_f32<TY, 2>), grid, dim3(256), 0, st, a);
+}
+
+static void launch_gemm_f32_args(hipStream_t st, GemmF32Args a) {
+  if (a.w.ty == RLH_TYPE_F32) a.n4 = 0;  // every token takes dot_f32_avx2 (ops.rs:165-174)
+  switch (a.w.ty) {
+    case RLH_TYPE_Q5_K: launch_f32_type<RLH_TYPE_Q5_K>(st, a); break;
+    case RLH_TYPE_Q4_1: launch_f32_type<RLH_TYPE_Q4_1>(st, a); break;
+    case RLH_TYPE_Q5_0: launch_f32_type<RLH_TYPE_Q5_0>(st, a); break;
+    case RLH_TYPE_Q5_1: launch_f32_type<RLH_TYPE_Q5_1>(st, a); break;
+    case RLH_TYPE_F16: launch_f32_type<RLH_TYPE_F16>(st, a); break;
+    case RLH_TYPE_BF16: launch_f32_type<RLH_TYPE_BF16>(st, a); break;
+    case RLH_TYPE_F32: launch_f32_type<RLH_TYPE_F32>(st, a); break;
+    default: break;
+  }
+}
+
 void launch_gemm_f32(hipStream_t st, const DevMat& w, const float* x, uint32_t n, uint32_t n4, float* y,
                      float* resid) {
   GemmF32Args a{};
@@ -777,18 +874,24 @@ void launch_gemm_f32(hipStream_t st, const DevMat& w, const float* x, uint32_t n
   a.n4 = n4;
   a.y = y;
   a.resid = resid;
-  if (w.ty == RLH_TYPE_F32) a.n4 = 0;  // every token takes dot_f32_avx2 (ops.rs:165-174)
-  const dim3 grid((w.rows + kFR - 1) / kFR, (n + kFT - 1) / kFT);
-  switch (w.ty) {
-    case RLH_TYPE_Q5_K: hipLaunchKernelGGL(k_gemm_f32<RLH_TYPE_Q5_K>, grid, dim3(256), 0, st, a); break;
-    case RLH_TYPE_Q4_1: hipLaunchKernelGGL(k_gemm_f32<RLH_TYPE_Q4_1>, grid, dim3(256), 0, st, a); break;
-    case RLH_TYPE_Q5_0: hipLaunchKernelGGL(k_gemm_f32<RLH_TYPE_Q5_0>, grid, dim3(256), 0, st, a); break;
-    case RLH_TYPE_Q5_1: hipLaunchKernelGGL(k_gemm_f32<RLH_TYPE_Q5_1>, grid, dim3(256), 0, st, a); break;
-    case RLH_TYPE_F16: hipLaunchKernelGGL(k_gemm_f32<RLH_TYPE_F16>, grid, dim3(256), 0, st, a); break;
-    case RLH_TYPE_BF16: hipLaunchKernelGGL(k_gemm_f32<RLH_TYPE_BF16>, grid, dim3(256), 0, st, a); break;
-    case RLH_TYPE_F32: hipLaunchKernelGGL(k_gemm_f32<RLH_TYPE_F32>, grid, dim3(256), 0, st, a); break;
-    default: break;
-  }
+  launch_gemm_f32_args(st, a);
+}
+
+bool gemm_f32_pair_supported(const DevMat& w, const DevMat& w2) {
+  return gemm_f32_supported(w.ty) && w2.ty == w.ty && w2.cols == w.cols;
+}
+
+void launch_gemm_f32_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const float* x, uint32_t n, uint32_t n4,
+                          float* y, float* y2) {
+  GemmF32Args a{};
+  a.w = w;
+  a.w2 = w2;
+  a.x = x;
+  a.n = n;
+  a.n4 = n4;
+  a.y = y;
+  a.y2 = y2;
+  launch_gemm_f32_args(st, a);
 }
 
 template <uint32_t TY>

@@ -17,7 +17,7 @@ import pytest
 
 import oracle
 import rlh
-from helpers import BF16, F16, F32, Q4_1, Q5_0, Q5_1, bits, random_blocks
+from helpers import BLOCK, BF16, F16, F32, Q4_1, Q5_0, Q5_1, bits, random_blocks
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +99,39 @@ def test_forward_bit_exact(name):
     c.close()
     oc.close()
     m.close()
+
+
+# The f32 products on MFMA at the edges of their jobs: only single tokens (n
+# < 4), groups of four with one to three single tokens left, the row tiles'
+# remainders (16-row blocks), and 32-row blocks (5500 rows x 131 tokens: 172
+# row tiles x 3 blocks).
+@pytest.mark.parametrize("ty", TYPES + [13], ids=[NAMES[t] for t in TYPES] + ["Q5_K"])
+@pytest.mark.parametrize("rows,cols,n", [(15, 256, 3), (17, 512, 4), (48, 768, 18), (65, 256, 67), (5500, 256, 131),
+                                         (16500, 512, 7)])
+def test_matmul_batch_job_edges_bit_exact(ty, rows, cols, n):
+    print(f"ty={ty} matmul_batch {rows}x{cols} n={n}", flush=True)
+    rng = np.random.default_rng(rows + cols * 5 + n + ty)
+    w = random_blocks(ty, rows * cols // BLOCK[ty][0], rng)
+    xs = rng.standard_normal((n, cols)).astype(np.float32)
+    got = rlh.matmul_batch(ty, w, rows, cols, xs, n)
+    ref = oracle.matmul_batch(ty, w, rows, cols, xs, n, oracle.MODE_BATCH_INT)
+    assert np.array_equal(bits(got), bits(ref))
+
+
+@pytest.mark.parametrize("ty", TYPES + [13], ids=[NAMES[t] for t in TYPES] + ["Q5_K"])
+def test_matmul_batch_non_finite_activations(ty):
+    """Infinite, NaN, subnormal and huge activations through the FMA chains."""
+    print(f"ty={ty} non-finite activations", flush=True)
+    rng = np.random.default_rng(ty)
+    rows, cols, n = 40, 512, 23
+    w = random_blocks(ty, rows * cols // BLOCK[ty][0], rng)
+    xs = rng.standard_normal((n, cols)).astype(np.float32)
+    for t, v in enumerate([np.inf, -np.inf, np.nan, 1e-41, 3e38, -3e38, 0.0]):
+        xs[3 * t, rng.integers(0, cols, 3)] = v
+    xs[21] *= np.float32(1e-38)
+    got = np.asarray(rlh.matmul_batch(ty, w, rows, cols, xs, n))
+    with np.errstate(all="ignore"):
+        ref = np.asarray(oracle.matmul_batch(ty, w, rows, cols, xs, n, oracle.MODE_BATCH_INT))
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(got[~nan].view(np.uint32), ref[~nan].view(np.uint32))
