@@ -15,12 +15,9 @@
 // (rmsnorm_head) and NeoX RoPE to the q heads and, in the block whose tile
 // holds the new position, to k, and writes K/V at pos (model.rs:642-656);
 // all of it in registers.
-// k_attn_qk_pre (prefill): one block per (KV head, 64-position tile, tile of
-// query tokens); lanes own positions as above, q reaches every lane by DPP
-// row broadcasts (below). Tiles above the causal diagonal exit at once.
-// k_attn_qk_pre_p (prefill, few blocks per CU): the same work items taken
-// by resident blocks in turn, the next item's K tile and q loaded while
-// the current one is computed.
+// k_attn_qk_pre (prefill): one block per (KV head, run of 32-position tiles,
+// tile of query tokens); the 32 chains of a dot product on the f32 MFMA
+// (below). Blocks above the causal diagonal exit at once.
 // k_attn_softmax: one block per (head, token): the row in LDS, max and exp
 // in parallel, the sequential sum in one lane, probabilities written back
 // over the scores.
@@ -239,293 +236,114 @@ __global__ void __launch_bounds__(256, 2) k_attn_qk(AttnArgs a) {
   }
 }
 
-// Prefill scores (q already normed and roped): k_attn_qk_pre (a block per
-// work item) or k_attn_qk_pre_p (persistent), below; a work item is (KV
-// head, 64-position tile, tile of combinations / G query tokens).
-constexpr int kPreQkComb = 64;  // k_attn_qk_pre: combinations per block (a multiple of 8)
-constexpr int kPreQkItem = 32;  // k_attn_qk_pre_p: combinations per work item (a multiple of 8)
-// k_attn_qk_pre_p runs when k_attn_qk_pre's blocks would fill at most this
-// many rounds of the resident blocks: it loads an item's K tile and q while
-// the previous item is computed, but each item waits for the previous one's
-// score stores to drain (one memory counter covers both), which costs more
-// than it saves once a block has many items (8B 512-token chunk, 2.25
-// rounds: 58 -> 43 us; 32B 4096-token chunks, 12-60 rounds: 468 -> 646 us)
-constexpr uint32_t kQkPersistRounds = 6;
-// blocks of k_attn_qk_pre_p the GPU holds at once (attn_init)
-uint32_t g_qk_pre_resident = 0;
+// Prefill scores (q already normed and roped) on the f32 MFMA, whose 16 x 16
+// x 4 product from C = 0 is, for every (position, combination) pair, the
+// chain fma(k_3, q_3, fma(.., fma(k_0, q_0, 0))): with element s + 32 k in
+// place of k it is slot s of dot_f32_avx2 exactly (simd.rs:328-377: 32 chains
+// of four). The slots then meet in the reference's tree, A_l = (slot l +
+// slot l+8) + (slot l+16 + slot l+24), ((A0+A4) + (A2+A6)) + ((A1+A5) +
+// (A3+A7)), on the VALU. Per 256 scores: 1024 cycles of MFMA and 31 x 4 adds;
+// one v_fma_f32 per element took 2000 cycles and the adds.
+//
+// A block takes T position tiles of 32 and kQkComb64 combinations
+// (token, query head) of a KV head, 16 per wave, whose q vectors stay in
+// registers (lane (k, i): elements 32 k .. + 31 of combination i). The K
+// tiles go to LDS by DMA, the next one while one is multiplied; 16-byte piece
+// p of row r sits at slot p ^ (r % 16) of its row, so that the 16 rows of an
+// operand read come from distinct banks. A lane ends up with four consecutive
+// scores of one combination. Four blocks per CU (32 positions staged at a
+// time, 110 registers). Average 512-token layer chunk of a 4096-token 32B
+// prompt: 445 us with v_fma_f32, 210 us (MFMA alone ~110).
+// grid: (KVH * ceil(tiles / T), ceil(n_tok / TP)), TP = 64 / G tokens;
+// block 256.
+constexpr uint32_t kQkComb64 = 64, kQkPos = 32;
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
-// acc[i] = fma(q_e, k_i, acc[i]) for the 8 elements e = 16m + R0 + i, whose
-// q_e is lane R0 + i of every row of 16 lanes in qm (v_fmac_f32 takes it by
-// DPP row_newbcast; one instruction per FMA, no broadcast copies). The
-// leading s_nop covers the DPP read-after-VALU-write hazard on qm.
-template <int R0>
-__device__ __forceinline__ void fmac8_bcast(float (&acc)[32], int s0, float qm, const f32x4_t& k0, const f32x4_t& k1) {
-  asm("s_nop 1\n\t"
-      "v_fmac_f32_dpp %0, %8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %8, %10 row_newbcast:%18 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %8, %11 row_newbcast:%19 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %8, %12 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %4, %8, %13 row_newbcast:%21 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %5, %8, %14 row_newbcast:%22 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %6, %8, %15 row_newbcast:%23 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %7, %8, %16 row_newbcast:%24 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc[s0]), "+v"(acc[s0 + 1]), "+v"(acc[s0 + 2]), "+v"(acc[s0 + 3]), "+v"(acc[s0 + 4]), "+v"(acc[s0 + 5]),
-        "+v"(acc[s0 + 6]), "+v"(acc[s0 + 7])
-      : "v"(qm), "v"(k0.x), "v"(k0.y), "v"(k0.z), "v"(k0.w), "v"(k1.x), "v"(k1.y), "v"(k1.z), "v"(k1.w), "i"(R0),
-        "i"(R0 + 1), "i"(R0 + 2), "i"(R0 + 3), "i"(R0 + 4), "i"(R0 + 5), "i"(R0 + 6), "i"(R0 + 7));
-}
-// step K of the 32 slot chains (elements s + 32K): slots 0..15 take qm[2K],
-// slots 16..31 qm[2K + 1]
-template <int K>
-__device__ __forceinline__ void qk_step(float (&acc)[32], const float (&qm)[8], const f32x4_t (&kreg)[32]) {
-  fmac8_bcast<0>(acc, 0, qm[2 * K], kreg[8 * K], kreg[8 * K + 1]);
-  fmac8_bcast<8>(acc, 8, qm[2 * K], kreg[8 * K + 2], kreg[8 * K + 3]);
-  fmac8_bcast<0>(acc, 16, qm[2 * K + 1], kreg[8 * K + 4], kreg[8 * K + 5]);
-  fmac8_bcast<8>(acc, 24, qm[2 * K + 1], kreg[8 * K + 6], kreg[8 * K + 7]);
-}
-
-// Work item of the persistent prefill scores kernel: KV head g, token tile y
-// (tokens y TP .. y TP + TP - 1) and a 64-position tile at or below the
-// tile's causal diagonal; per KV head the items run y-major. count(y) is
-// the number of position tiles token tile y sees.
-struct QkItem {
-  uint32_t g, tile, tok0, ntok;
-};
-__host__ __device__ inline uint32_t qk_tiles_seen(uint32_t p0, uint32_t n_tok, uint32_t TP, uint32_t y) {
-  const uint32_t last = p0 + (n_tok < (y + 1) * TP ? n_tok : (y + 1) * TP) - 1;
-  return last / kPosTile + 1;
-}
-__host__ __device__ inline uint32_t qk_items_per_head(uint32_t p0, uint32_t n_tok, uint32_t TP) {
-  uint32_t n = 0;
-  for (uint32_t y = 0; y * TP < n_tok; y++) n += qk_tiles_seen(p0, n_tok, TP, y);
-  return n;
-}
-__device__ inline QkItem qk_item(uint32_t it, uint32_t per_g, uint32_t p0, uint32_t n_tok, uint32_t TP) {
-  QkItem q;
-  q.g = it / per_g;
-  uint32_t r = it % per_g, y = 0;
-  for (;; y++) {  // r < per_g: some token tile holds it
-    const uint32_t c = qk_tiles_seen(p0, n_tok, TP, y);
-    if (r < c) break;
-    r -= c;
-  }
-  q.tile = r;
-  q.tok0 = y * TP;
-  q.ntok = n_tok - q.tok0 < TP ? n_tok - q.tok0 : TP;
-  return q;
-}
-
-// Prefill scores (q already normed and roped): one block per (KV head,
-// 64-position tile, tile of kPreQkComb / G query tokens). The K tile is
-// staged in LDS once and each lane (= position) keeps its K row in
-// registers. The wave walks its (token, head) combinations with q held in
-// every row of 16 lanes (lane r of a row holds elements 16m + r in qm[m])
-// and broadcast to the row by DPP (row_newbcast), so no q element passes
-// through LDS; the next combination's q is loaded while the current one is
-// computed. Slot s (0..31) of dot_f32_avx2 is the FMA chain over elements s,
-// s+32, s+64, s+96, A_l = (slot l + slot l+8) + (slot l+16 + slot l+24),
-// then the AVX2 tree (simd.rs:328-377).
-// grid: (KVH * ntiles, ceil(n_tok / TP)), TP = kPreQkComb / G; block 256.
-__global__ void __launch_bounds__(256, 2) k_attn_qk_pre(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) float kt_g[kPosTile * kKStride];
-  __shared__ __attribute__((aligned(16))) float qv_g[kPreQkComb * kHd];
+__global__ void __launch_bounds__(256, 4) k_attn_qk_pre(AttnArgs a, uint32_t T) {
+  __shared__ __attribute__((aligned(16))) float kt_g[2][kQkPos * kHd];
   lfloat* kt = (lfloat*)kt_g;
-  lfloat* qv = (lfloat*)qv_g;
-  const uint32_t G = (uint32_t)(a.H / a.KVH), TP = (uint32_t)kPreQkComb / G;
-  const uint32_t ntiles = (a.t_max + kPosTile - 1) / kPosTile;
-  const uint32_t g = blockIdx.x / ntiles, tile = blockIdx.x % ntiles;
+  const uint32_t G = (uint32_t)(a.H / a.KVH), TP = kQkComb64 / G;
+  const uint32_t ntiles = (a.t_max + kQkPos - 1) / kQkPos, nsplit = (ntiles + T - 1) / T;
+  const uint32_t g = blockIdx.x / nsplit, tile0 = blockIdx.x % nsplit * T;
   const uint32_t tok0 = blockIdx.y * TP;
-  const uint32_t ntok = a.n_tok - tok0 < TP ? a.n_tok - tok0 : TP;
+  const uint32_t ntok = a.n_tok - tok0 < TP ? a.n_tok - tok0 : TP, ncomb = ntok * G;
   const uint32_t pos_first = a.pos0[0] + tok0, pos_last = pos_first + ntok - 1;
-  const uint32_t j0 = tile * kPosTile;
-  if (j0 > pos_last) return;  // whole tile above the causal diagonal
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tile0 * kQkPos > pos_last) return;  // whole block above the causal diagonal
+  const uint32_t nt = min(T, pos_last / kQkPos + 1 - tile0);
+  const uint32_t lane = threadIdx.x & 63, l = lane & 15, q = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t qd = (uint32_t)a.H * kHd, kvd = (uint32_t)a.KVH * kHd;
-  // K tile rows in natural element order (rows past pos_last repeat it)
-  float4 kr[8];
+  // the lane's combination (as the MFMA's column), its q vector and row of scores
+  const uint32_t c = 16 * wave + l, tt = min(c, ncomb - 1) / G, h = g * G + min(c, ncomb - 1) % G;
+  const float* qp = a.q + (size_t)(tok0 + tt) * qd + h * kHd + 32 * q;
+  f32x4_t qf[8];
 #pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const uint32_t c = tid + 256u * i, jl = c >> 5, f4 = c & 31, j = min(j0 + jl, pos_last);
-    kr[i] = ld_gf4(a.kcache + (size_t)j * kvd + g * kHd + 4 * f4);
-  }
-  // combinations of tokens that see at least one position of the tile;
-  // the wave's first q is loaded with the K tile
-  const uint32_t tt0 = j0 > pos_first ? j0 - pos_first : 0u;
-  const uint32_t ncomb = ntok * G;
-  // the block's q vectors are staged in LDS with the K tile, element
-  // 16 m + r of a combination at r * 8 + m, so that lane r of every row of
-  // 16 lanes reads its eight elements in two 16-byte reads
-  constexpr int kQv = kPreQkComb / 8;  // float4s of q per thread (32 per combination)
-  float4 qr[kQv];
+  for (int i = 0; i < 8; i++) qf[i] = *(const RLH_GLOBAL f32x4_t*)(qp + 4 * i);
+  float* out = a.scores + ((size_t)(tok0 + tt) * a.H + h) * a.t_stride;
+  const uint32_t seen = c < ncomb ? pos_first + tt + 1 : 0;  // positions the combination sees
+  // the wave's first and last tokens' positions (a wave past the last
+  // combination only copies)
+  const bool live = 16 * wave < ncomb;
+  const uint32_t wave_first = pos_first + 16 * wave / G, wave_last = pos_first + min(16 * wave + 15, ncomb - 1) / G;
+  const bool whole = 16 * wave + 15 < ncomb;
+  auto dma = [&](uint32_t t) {  // rows past pos_last repeat it
 #pragma unroll
-  for (int i = 0; i < kQv; i++) {
-    const uint32_t ci = tid + 256u * i, cb = min(ci >> 5, ncomb - 1), f4 = ci & 31;
-    qr[i] = ld_gf4(a.q + (size_t)(tok0 + cb / G) * qd + (g * G + cb % G) * kHd + 4 * f4);
-  }
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const uint32_t ci = tid + 256u * i, jl = ci >> 5, f4 = ci & 31;
-    *(lf32x4*)(kt + jl * kKStride + 4 * f4) = f32x4_t{kr[i].x, kr[i].y, kr[i].z, kr[i].w};
-  }
-#pragma unroll
-  for (int i = 0; i < kQv; i++) {
-    const uint32_t ci = tid + 256u * i, cb = ci >> 5, f4 = ci & 31;  // cb < kPreQkComb
-    lfloat* qd0 = qv + cb * kHd + 4 * (f4 & 3) * 8 + (f4 >> 2);
-    qd0[0] = qr[i].x;
-    qd0[8] = qr[i].y;
-    qd0[16] = qr[i].z;
-    qd0[24] = qr[i].w;
-  }
-  auto q_load = [&](float (&qm)[8], uint32_t c) {
-    const lf32x4* qp = (const lf32x4*)(qv + min(c, ncomb - 1) * kHd + (lane & 15) * 8);
-    const f32x4_t u0 = qp[0], u1 = qp[1];
-    qm[0] = u0.x, qm[1] = u0.y, qm[2] = u0.z, qm[3] = u0.w;
-    qm[4] = u1.x, qm[5] = u1.y, qm[6] = u1.z, qm[7] = u1.w;
+    for (uint32_t n = 0; n < kQkPos / 8; n++) {
+      const uint32_t r = 2 * (kQkPos / 8 * wave + n) + lane / 32, p = (lane & 31) ^ (r & 15);
+      const uint32_t j = min((tile0 + t) * kQkPos + r, pos_last);
+      __builtin_amdgcn_global_load_lds((const RLH_GLOBAL void*)(a.kcache + (size_t)j * kvd + g * kHd + 4 * p),
+                                       (RLH_LDS void*)(kt + (t & 1) * (kQkPos * kHd) + (kQkPos / 8 * wave + n) * 256), 16, 0,
+                                       0);
+    }
   };
-  float qa[8], qb[8];
-  uint32_t c = tt0 * G + wave;
-  __syncthreads();
-  q_load(qa, c);
-  const uint32_t j = j0 + lane;
-  f32x4_t kreg[32];
+  // slots of the lane's pieces 8 q .. 8 q + 7 in a row r = l (mod 16)
+  uint32_t slot[8];
 #pragma unroll
-  for (int i = 0; i < 32; i++) kreg[i] = *(const lf32x4*)(kt + lane * kKStride + 4 * i);
-  auto one = [&](const float (&qm)[8], uint32_t cc) {
-    const uint32_t tt = cc / G, h = g * G + cc % G;
-    float acc[32];
-#pragma unroll
-    for (int s = 0; s < 32; s++) acc[s] = 0.0f;  // fma(q, k, +0) starts each chain, as the reference
-    qk_step<0>(acc, qm, kreg);
-    qk_step<1>(acc, qm, kreg);
-    qk_step<2>(acc, qm, kreg);
-    qk_step<3>(acc, qm, kreg);
-    float A[8];
-#pragma unroll
-    for (int l = 0; l < 8; l++) A[l] = (acc[l] + acc[l + 8]) + (acc[l + 16] + acc[l + 24]);
-    const float d = ((A[0] + A[4]) + (A[2] + A[6])) + ((A[1] + A[5]) + (A[3] + A[7]));
-    if (j <= pos_first + tt) a.scores[((size_t)(tok0 + tt) * a.H + h) * a.t_stride + j] = d * a.scale;
-  };
+  for (uint32_t i = 0; i < 8; i++) slot[i] = l * kHd + 4 * ((8 * q + i) ^ l);
+  dma(0);
+  bool stored = false;  // the last tile ended with exactly four stores of this wave
+  for (uint32_t t = 0; t < nt; t++) {
+    // tile t has landed (its copies were issued before the last tile's
+    // stores, which need not be waited for); past the barrier every wave is
+    // done with the other buffer
+    if (stored)
+      wait_vmcnt<kQkPos / 16>();
+    else
+      wait_vmcnt<0>();
+    lds_barrier();
+    if (t + 1 < nt) dma(t + 1);
+    const uint32_t j0 = (tile0 + t) * kQkPos;
+    stored = false;
+    if (!live || j0 > wave_last) continue;
+    const lfloat* kb = kt + (t & 1) * (kQkPos * kHd);
+    const bool full = whole && j0 + kQkPos - 1 <= wave_first;  // every lane sees the whole tile
 #pragma unroll 1
-  for (; c < ncomb; c += 8) {
-    q_load(qb, c + 4);
-    one(qa, c);
-    if (c + 4 >= ncomb) break;
-    q_load(qa, c + 8);
-    one(qb, c + 4);
-  }
-}
-
-// grid: the resident blocks (at most the items); block 256. Block b takes
-// items b, b + gridDim.x, ... (exits are uniform, no waits between blocks).
-// Per item the K tile is staged in LDS and each lane (= position) keeps its
-// K row in registers; the item's q vectors sit in one of two LDS buffers in
-// their natural element order, copied there by DMA. While an item is
-// computed, the next item's K tile is loaded into registers and its q
-// vectors are copied into the other buffer, so the loads' latency is paid
-// once per block instead of once per item; the combination loop issues no
-// global loads (nothing it waits for queues behind the next item's). Lane
-// r of every row of 16 lanes reads elements 16 m + r of q (conflict-free
-// 4-byte reads) into qm[m], which the FMAs take by DPP row broadcasts
-// (fmac8_bcast). Slot s (0..31) of dot_f32_avx2 is the FMA chain over
-// elements s, s+32, s+64, s+96, A_l = (slot l + slot l+8) + (slot l+16 +
-// slot l+24), then the AVX2 tree (simd.rs:328-377).
-__global__ void __launch_bounds__(256, 2) k_attn_qk_pre_p(AttnArgs a, uint32_t per_g) {
-  __shared__ __attribute__((aligned(16))) float kt_g[kPosTile * kKStride];
-  __shared__ __attribute__((aligned(16))) float qv_g[2][kPreQkItem * kHd];
-  lfloat* kt = (lfloat*)kt_g;
-  const uint32_t G = (uint32_t)(a.H / a.KVH), TP = (uint32_t)kPreQkItem / G;
-  const uint32_t p0h = a.t_max - a.n_tok;  // the chunk's first position (the host's view of pos0)
-  const uint32_t n_items = (uint32_t)a.KVH * per_g;
-  uint32_t it = blockIdx.x;
-  if (it >= n_items) return;  // whole block, before any barrier
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t qd = (uint32_t)a.H * kHd, kvd = (uint32_t)a.KVH * kHd;
-  const uint32_t p0 = a.pos0[0];
-  // an item's K tile rows in natural element order (rows past its last
-  // token's position repeat that row)
-  auto load_k = [&](float4 (&kr)[8], const QkItem& q) {
-    const uint32_t pos_last = p0 + q.tok0 + q.ntok - 1, j0 = q.tile * kPosTile;
+    for (uint32_t st = 0; st < kQkPos / 16; st++) {
+      f32x4_t kv[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const uint32_t c = tid + 256u * i, jl = c >> 5, f4 = c & 31, j = min(j0 + jl, pos_last);
-      kr[i] = ld_gf4(a.kcache + (size_t)j * kvd + q.g * kHd + 4 * f4);
+      for (int i = 0; i < 8; i++) kv[i] = *(const lf32x4*)(kb + st * 16 * kHd + slot[i]);
+      auto chain = [&](int s) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(kv[s / 4][s % 4], qf[s / 4][s % 4], f32x4_t{}, 0, 0, 0);
+      };
+      auto A = [&](int i) {
+        const f32x4_t s0 = chain(i), s1 = chain(i + 8), s2 = chain(i + 16), s3 = chain(i + 24);
+        return (s0 + s1) + (s2 + s3);
+      };
+      const f32x4_t e0 = A(0) + A(4);
+      const f32x4_t e = e0 + (A(2) + A(6));
+      const f32x4_t o0 = A(1) + A(5);
+      const f32x4_t o = o0 + (A(3) + A(7));
+      const f32x4_t d = (e + o) * a.scale;
+      const uint32_t j = j0 + 16 * st + 4 * q;
+      if (full) {
+        *(RLH_GLOBAL f32x4u_t*)(out + j) = d;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (j + i < seen) ((RLH_GLOBAL float*)out)[j + i] = d[i];
+      }
     }
-  };
-  // an item's q vectors into buffer b by DMA: one 1 KB copy per wave and
-  // step holds two combinations (lanes 0..31 and 32..63, 16 bytes each);
-  // combinations past the last token repeat the last one
-  auto dma_q = [&](uint32_t b, const QkItem& q) {
-    const uint32_t ncomb = q.ntok * G;
-#pragma unroll
-    for (uint32_t k = 0; k < (uint32_t)kPreQkItem / 8; k++) {
-      const uint32_t pair = wave + 4 * k, cb = min(2 * pair + lane / 32, ncomb - 1);
-      __builtin_amdgcn_global_load_lds(
-          (const RLH_GLOBAL void*)(a.q + (size_t)(q.tok0 + cb / G) * qd + (q.g * G + cb % G) * kHd + 4 * (lane % 32)),
-          (RLH_LDS void*)((lfloat*)qv_g[b] + 2 * pair * kHd), 16, 0, 0);
-    }
-  };
-  QkItem cur = qk_item(it, per_g, p0h, a.n_tok, TP);
-  float4 kr[8];
-  load_k(kr, cur);
-  dma_q(0, cur);
-  for (uint32_t n = 0;; n++) {
-    wait_vmcnt<0>();  // this wave's K rows and q copies of the item have landed
-    __syncthreads();  // ... everyone's; every wave is done with the previous kt
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const uint32_t ci = tid + 256u * i, jl = ci >> 5, f4 = ci & 31;
-      *(lf32x4*)(kt + jl * kKStride + 4 * f4) = f32x4_t{kr[i].x, kr[i].y, kr[i].z, kr[i].w};
-    }
-    __syncthreads();
-    f32x4_t kreg[32];
-#pragma unroll
-    for (int i = 0; i < 32; i++) kreg[i] = *(const lf32x4*)(kt + lane * kKStride + 4 * i);
-    const lfloat* qv = (const lfloat*)qv_g[n & 1];
-    const uint32_t nit = it + gridDim.x;
-    const bool more = nit < n_items;
-    QkItem nxt = cur;
-    if (more) {  // uniform: the next item's K tile and q vectors in flight
-      nxt = qk_item(nit, per_g, p0h, a.n_tok, TP);
-      load_k(kr, nxt);
-      dma_q((n + 1) & 1, nxt);  // that buffer's last reader was the item before this one
-    }
-    const uint32_t j0 = cur.tile * kPosTile, pos_first = p0 + cur.tok0, ncomb = cur.ntok * G;
-    const uint32_t j = j0 + lane;
-    auto q_load = [&](float (&qm)[8], uint32_t c) {
-      const lfloat* qp = qv + min(c, ncomb - 1) * kHd + (lane & 15);
-#pragma unroll
-      for (int m = 0; m < 8; m++) qm[m] = qp[16 * m];
-    };
-    auto one = [&](const float (&qm)[8], uint32_t cc) {
-      const uint32_t tt = cc / G, h = cur.g * G + cc % G;
-      float acc[32];
-#pragma unroll
-      for (int s = 0; s < 32; s++) acc[s] = 0.0f;  // fma(q, k, +0) starts each chain, as the reference
-      qk_step<0>(acc, qm, kreg);
-      qk_step<1>(acc, qm, kreg);
-      qk_step<2>(acc, qm, kreg);
-      qk_step<3>(acc, qm, kreg);
-      float A[8];
-#pragma unroll
-      for (int l = 0; l < 8; l++) A[l] = (acc[l] + acc[l + 8]) + (acc[l + 16] + acc[l + 24]);
-      const float d = ((A[0] + A[4]) + (A[2] + A[6])) + ((A[1] + A[5]) + (A[3] + A[7]));
-      if (j <= pos_first + tt) a.scores[((size_t)(cur.tok0 + tt) * a.H + h) * a.t_stride + j] = d * a.scale;
-    };
-    // tokens before tt0 see no position of the tile
-    uint32_t c = (j0 > pos_first ? j0 - pos_first : 0u) * G + wave;
-    float qa[8], qb[8];
-    q_load(qa, c);
-#pragma unroll 1
-    for (; c < ncomb; c += 8) {
-      q_load(qb, c + 4);
-      one(qa, c);
-      if (c + 4 >= ncomb) break;
-      q_load(qa, c + 8);
-      one(qb, c + 4);
-    }
-    if (!more) break;
-    it = nit;
-    cur = nxt;
+    stored = full;
   }
 }
 
@@ -1532,17 +1350,20 @@ void launch_attn_scores(hipStream_t st, const AttnArgs& a, bool fused) {
   if (fused) {
     hipLaunchKernelGGL(k_attn_qk, dim3(a.KVH * ntiles, a.n_tok), dim3(256), 0, st, a);
   } else {
-    const uint32_t G = (uint32_t)(a.H / a.KVH), p0 = a.t_max - a.n_tok;
-    const uint32_t TP = (uint32_t)kPreQkComb / G, blocks = (uint32_t)a.KVH * qk_items_per_head(p0, a.n_tok, TP);
-    const char* env = std::getenv("RLH_QK_PRE_GRID");  // '1': always the grid kernel (tests)
-    const bool grid_only = env && env[0] == '1';
-    if (!grid_only && g_qk_pre_resident && blocks <= kQkPersistRounds * g_qk_pre_resident) {
-      const uint32_t per_g = qk_items_per_head(p0, a.n_tok, (uint32_t)kPreQkItem / G);
-      const uint32_t n_items = (uint32_t)a.KVH * per_g;
-      hipLaunchKernelGGL(k_attn_qk_pre_p, dim3(std::min(n_items, g_qk_pre_resident)), dim3(256), 0, st, a, per_g);
-    } else {
-      hipLaunchKernelGGL(k_attn_qk_pre, dim3(a.KVH * ntiles, (a.n_tok + TP - 1) / TP), dim3(256), 0, st, a);
+    const uint32_t TP = kQkComb64 / (uint32_t)(a.H / a.KVH), p0 = a.t_max - a.n_tok, ntiles = (a.t_max + kQkPos - 1) / kQkPos;
+    // the most tiles per block (one q load for all of them) that leave 512
+    // blocks with work; us by T = 8 / 4 / 2 / 1: 32B, 512 tokens up to 4096
+    // positions 210 / 215 / 228 / 276; 8B, 61 after 700 30 / 21 / 20 / 20;
+    // 0.6B, 48 7.4 / 7.6 / 7.3 / 5.8
+    uint32_t T = 8;
+    for (; T > 1; T /= 2) {
+      uint32_t blocks = 0;
+      for (uint32_t y = 0; y * TP < a.n_tok; y++)
+        blocks += (p0 + std::min(a.n_tok, (y + 1) * TP) - 1) / kQkPos / T + 1;
+      if (blocks * (uint32_t)a.KVH >= 512) break;
     }
+    hipLaunchKernelGGL(k_attn_qk_pre, dim3(a.KVH * ((ntiles + T - 1) / T), (a.n_tok + TP - 1) / TP), dim3(256), 0, st,
+                       a, T);
   }
 }
 
@@ -1606,14 +1427,6 @@ void launch_attn_pv(hipStream_t st, const AttnArgs& a, bool decode) {
 
 bool attn_init(uint32_t max_ctx) {
   if (max_ctx > kAttnMaxCtx) return false;
-  if (!g_qk_pre_resident) {
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_attn_qk_pre_p, 256, 0) == hipSuccess &&
-        cus > 0 && per_cu > 0)
-      g_qk_pre_resident = (uint32_t)(cus * per_cu);
-  }
   size_t ring_lds = 0;
   for (uint32_t gq = 1; gq <= (uint32_t)kAttnMaxGroup; gq++) ring_lds = std::max(ring_lds, pv_ring_lds(gq));
   return hipFuncSetAttribute((const void*)k_attn_softmax<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
