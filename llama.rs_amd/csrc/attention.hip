@@ -56,8 +56,6 @@ __host__ __device__ constexpr uint32_t softmax_rows_stride(uint32_t t_max) { ret
 constexpr int kKStride = 132;   // floats per staged K row (permuted + 4 pad)
 constexpr int kQkComb = 16;     // (token, head) combinations per scores block
 constexpr int kDecChunk = 256;  // positions per LDS chunk, decode PV
-constexpr int kPreChunk = 64;   // positions per LDS chunk, prefill PV
-constexpr int kPreComb = 32;    // (token, head) combinations per prefill PV block
 // dynamic LDS of the fused decode kernel's score rows (its V chunks take
 // 66.5 KB of static LDS)
 constexpr size_t kDecFusedLds = 88u * 1024u;
@@ -1226,111 +1224,127 @@ __global__ void __launch_bounds__(512) k_attn_pv_ring(AttnArgs a) {
   }
 }
 
-// grid: (KVH, ceil(n_tok / TT)), TT = 32 / G tokens per block, latest (most
-// positions) token tiles first; block 512: thread (d = tid % 128, quarter
-// tid / 128) runs the chains of combinations quarter + 4i.
-__global__ void __launch_bounds__(512) k_attn_pv_pre(AttnArgs a) {
-  constexpr int CS = kPreChunk + 4;
-  constexpr int NC = kPreComb / 4;  // chains per thread
-  __shared__ __attribute__((aligned(16))) float vs_g[kPreChunk * kHd];
-  __shared__ __attribute__((aligned(16))) float ps_g[kPreComb * CS];
-  lfloat* vs = (lfloat*)vs_g;
-  lfloat* ps = (lfloat*)ps_g;
-  const int G = a.H / a.KVH;
-  const uint32_t TT = (uint32_t)(kPreComb / G);
-  const int ncomb = (int)TT * G;
-  const uint32_t g = blockIdx.x;
+// Prefill: the ordered sums o_d = p_j * V_j[d] + o_d of every combination
+// (token, query head). The products come from the f32 MFMA: a 16 x 16 x 1
+// product in four blocks from C = 0 is round(p_j * V_j[d]) for 16
+// combinations x 16 d x 4 positions, in 32 cycles where 16 v_mul_f32 take 37;
+// above all its operands are one value per lane, where the VALU form reads
+// every probability as a 16-byte broadcast and was bound by those reads. The
+// adds stay on the VALU, position by position. (A product of -0 comes back as
+// +0: the sums start at +0 and never become -0, so neither changes them.)
+//
+// Block: 16 combinations of a KV head x 16 NW d, NW waves of 16 d. V rows and
+// probabilities come to LDS by DMA, 32 positions at a time, the next chunk
+// while one is summed (three or four chunks in LDS measured slower: fewer
+// blocks per CU); position j of combination c sits at slot j ^ c of its 32,
+// so that an operand read hits distinct banks. At the end the sums pass
+// through LDS into Q8 blocks. Average 512-token layer chunk of a 4096-token
+// 32B prompt: 402 us with v_mul_f32, 323 us (the products and adds alone
+// 237); 8B 512 tokens 52, 40; 61 after 700 52, 30; 0.6B 48 15.6, 6.1. Two
+// tiles of combinations or of d per wave were no faster.
+// grid: (KVH, ceil(n_tok / TT), 8 / NW), TT = 16 / G tokens per block, latest
+// (most positions) token tiles first; block 64 NW.
+constexpr uint32_t kPvPos = 32, kPvComb = 16;  // positions per chunk, combinations per block
+// words of a chunk: V rows of 16 NW d, then probabilities
+constexpr uint32_t pv_pre_words(uint32_t nw) { return kPvPos * (16 * nw + kPvComb); }
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) k_attn_pv_pre(AttnArgs a) {
+  constexpr uint32_t kD = 16 * NW, kPvWords = pv_pre_words(NW), kRows = 256 / kD;  // d, LDS words, V rows per copy
+  __shared__ __attribute__((aligned(16))) float lds_g[2 * kPvWords];
+  lfloat* lds = (lfloat*)lds_g;
+  const uint32_t G = (uint32_t)(a.H / a.KVH), TT = kPvComb / G, g = blockIdx.x, dbase = kD * blockIdx.z;
   const uint32_t tok0 = (gridDim.y - 1 - blockIdx.y) * TT;
-  const uint32_t ntok = a.n_tok - tok0 < TT ? a.n_tok - tok0 : TT;
-  const int tid = threadIdx.x, d = tid & 127, qtr = tid >> 7;
-  const int qd = a.H * kHd, kvd = a.KVH * kHd;
-  const uint32_t p0 = a.pos0[0];
-  const uint32_t t_lo = p0 + tok0 + 1, t_hi = p0 + tok0 + ntok;
-  float o[NC];
-  uint32_t tlim[NC];  // positions chain i takes (0 for combinations past the last token)
+  const uint32_t ntok = a.n_tok - tok0 < TT ? a.n_tok - tok0 : TT, ncomb = ntok * G;
+  const uint32_t lane = threadIdx.x & 63, l = lane & 15, q = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t qd = (uint32_t)a.H * kHd, kvd = (uint32_t)a.KVH * kHd;
+  const uint32_t p0 = a.pos0[0], t_lo = p0 + tok0 + 1, t_hi = p0 + tok0 + ntok;
+  const uint32_t nch = (t_hi + kPvPos - 1) / kPvPos;
+  // the wave's copies of a chunk: two of V rows and 8 / NW of two
+  // combinations each (indices clamped into the rows that hold values)
+  constexpr uint32_t kPCopies = 8 / NW;
+  const float* vcol = a.vcache + g * kHd + dbase + 4 * (lane % (kD / 4));
+  auto dma = [&](uint32_t ch) {
+    lfloat* b = lds + (ch & 1) * kPvWords;
+    const uint32_t j0 = ch * kPvPos;
 #pragma unroll
-  for (int i = 0; i < NC; i++) {
-    o[i] = 0.0f;
-    const int cb = qtr + 4 * i;
-    const uint32_t tt = (uint32_t)(cb / G);
-    tlim[i] = cb < ncomb && tt < ntok ? p0 + tok0 + tt + 1 : 0u;
-  }
-  // chunk loads go to registers one chunk ahead and into LDS after the
-  // chunk in use is consumed
-  float4 vr[4];
-  float pr[4];
-  auto load = [&](uint32_t j0) {
-    const uint32_t jn = t_hi - j0 < (uint32_t)kPreChunk ? t_hi - j0 : (uint32_t)kPreChunk;
+    for (uint32_t n = 0; n < 2; n++) {
+      const uint32_t i = 2 * wave + n, j = min(j0 + kRows * i + lane / (kD / 4), t_hi - 1);
+      __builtin_amdgcn_global_load_lds((const RLH_GLOBAL void*)(vcol + (size_t)j * kvd), (RLH_LDS void*)(b + i * 256),
+                                       16, 0, 0);
+    }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {  // unconditional: indices clamped into bounds
-      const uint32_t c = (uint32_t)(tid + 512 * i), jl = c >> 5, f4 = c & 31;
-      vr[i] = ld_gf4(a.vcache + (size_t)(j0 + min(jl, jn - 1)) * kvd + g * kHd + 4 * f4);
-      const uint32_t cb = min(c / kPreChunk, (uint32_t)ncomb - 1), pl = c % kPreChunk;
-      const uint32_t tt = min(cb / G, ntok - 1);
-      pr[i] = ld_gf(a.scores + ((size_t)(tok0 + tt) * a.H + g * G + cb % G) * a.t_stride +
-                    min(j0 + pl, p0 + tok0 + tt));
+    for (uint32_t n = 0; n < kPCopies; n++) {
+      const uint32_t i = kPCopies * wave + n, r = 2 * i + lane / 32, c = min(r, ncomb - 1), tok = tok0 + c / G;
+      __builtin_amdgcn_global_load_lds(
+          (const RLH_GLOBAL void*)(a.scores + ((size_t)tok * a.H + g * G + c % G) * a.t_stride +
+                                   min(j0 + ((lane ^ r) & 31), p0 + tok)),
+          (RLH_LDS void*)(b + kPvPos * kD + i * 64), 4, 0, 0);
     }
   };
-  auto store = [&](uint32_t j0) {
-    const uint32_t jn = t_hi - j0 < (uint32_t)kPreChunk ? t_hi - j0 : (uint32_t)kPreChunk;
+  f32x4_t o = {};  // combination 4 q + e, d = 16 wave + l
+  dma(0);
+  for (uint32_t ch = 0; ch < nch; ch++) {
+    wait_vmcnt<0>();  // this wave's copies of the chunk have landed
+    lds_barrier();    // ... everyone's; every wave is done with the other buffer
+    if (ch + 1 < nch) dma(ch + 1);
+    const uint32_t j0 = ch * kPvPos;
+    const lfloat* vb = lds + (ch & 1) * kPvWords + q * kD + 16 * wave + l;
+    const lfloat* pb = lds + (ch & 1) * kPvWords + kPvPos * kD + l * kPvPos;
+    // the products of positions jj .. jj + 3 (lane group q: position jj + q)
+    auto products = [&](uint32_t jj) {
+      return __builtin_amdgcn_mfma_f32_16x16x1f32(pb[(jj + q) ^ l], vb[jj * kD], f32x16_t{}, 0, 0, 0);
+    };
+    auto add = [&](const f32x16_t& pr) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t c = (uint32_t)(tid + 512 * i), jl = c >> 5, f4 = c & 31;
-      if (jl < jn) *(lf32x4*)(vs + jl * kHd + 4 * f4) = f32x4_t{vr[i].x, vr[i].y, vr[i].z, vr[i].w};
-      const uint32_t cb = c / kPreChunk, pl = c % kPreChunk, tt = cb / G;
-      if ((int)cb < ncomb && tt < ntok && j0 + pl < p0 + tok0 + tt + 1) ps[cb * CS + pl] = pr[i];
+      for (int b = 0; b < 4; b++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = pr[4 * b + e] + o[e];
+    };
+    if (j0 + kPvPos <= t_lo) {  // every combination sees the whole chunk
+      // (the operands of the next products are read before these are summed)
+      float p[2], v[2];
+      auto read = [&](uint32_t s) { p[s & 1] = pb[(4 * s + q) ^ l], v[s & 1] = vb[4 * s * kD]; };
+      read(0);
+#pragma unroll
+      for (uint32_t s = 0; s < kPvPos / 4; s++) {
+        if (s + 1 < kPvPos / 4) read(s + 1);
+        const f32x16_t pr = __builtin_amdgcn_mfma_f32_16x16x1f32(p[s & 1], v[s & 1], f32x16_t{}, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        add(pr);
+      }
+      continue;
     }
-  };
-  load(0);
-  store(0);
-  __syncthreads();
-  for (uint32_t j0 = 0; j0 < t_hi; j0 += kPreChunk) {
-    const uint32_t jn = t_hi - j0 < (uint32_t)kPreChunk ? t_hi - j0 : (uint32_t)kPreChunk;
-    const bool more = j0 + kPreChunk < t_hi;
-    if (more) load(j0 + kPreChunk);
-    // positions below t_lo are taken by every chain
-    const uint32_t jf = t_lo > j0 ? (t_lo - j0 < jn ? t_lo - j0 : jn) : 0u;
-    // every chain runs here, branch-free, with all its p reads issued before
-    // the arithmetic (a chain past the last token reads rows of ps that hold
-    // nothing and is never stored)
-    uint32_t jj = 0;
-    for (; jj + 4 <= jf; jj += 4) {
-      const float v0 = vs[jj * kHd + d], v1 = vs[(jj + 1) * kHd + d];
-      const float v2 = vs[(jj + 2) * kHd + d], v3 = vs[(jj + 3) * kHd + d];
-      f32x4_t p[NC];
+    for (uint32_t jj = 0; jj < min(t_hi - j0, kPvPos); jj += 4) {
+      const f32x16_t pr = products(jj);
 #pragma unroll
-      for (int i = 0; i < NC; i++) p[i] = *(const lf32x4*)(ps + (qtr + 4 * i) * CS + jj);
+      for (int e = 0; e < 4; e++) {  // each combination takes the positions it sees
+        const uint32_t seen = t_lo + min(4 * q + e, ncomb - 1) / G;
 #pragma unroll
-      for (int i = 0; i < NC; i++) {
-        o[i] = p[i].x * v0 + o[i];
-        o[i] = p[i].y * v1 + o[i];
-        o[i] = p[i].z * v2 + o[i];
-        o[i] = p[i].w * v3 + o[i];
+        for (int b = 0; b < 4; b++) o[e] = j0 + jj + b < seen ? pr[4 * b + e] + o[e] : o[e];
       }
     }
-    for (; jj < jn; jj++) {
-      const uint32_t j = j0 + jj;
-      const float v = vs[jj * kHd + d];
-#pragma unroll
-      for (int i = 0; i < NC; i++)
-        if (j < tlim[i]) o[i] = ps[(qtr + 4 * i) * CS + jj] * v + o[i];
-    }
-    __syncthreads();  // the chunk is consumed
-    if (more) {
-      store(j0 + kPreChunk);
-      __syncthreads();
-    }
   }
+  // the sums to LDS [combination][d], then 32 d per half wave: the f32 row
+  // and its Q8 blocks
+  lds_barrier();
 #pragma unroll
-  for (int i = 0; i < NC; i++) {
-    if (tlim[i]) {
-      const int cb = qtr + 4 * i;
-      const uint32_t tok = tok0 + (uint32_t)(cb / G);
-      const uint32_t col = (uint32_t)(g * G + cb % G) * kHd + d;
-      ((RLH_GLOBAL float*)a.out)[(size_t)tok * qd + col] = o[i];
-      q8_quant_block32(o[i], a.out_tiles, tok, col / 32);
-    }
+  for (int e = 0; e < 4; e++) lds[(4 * q + e) * kD + 16 * wave + l] = o[e];
+  lds_barrier();
+  for (uint32_t i = threadIdx.x; i < ncomb * kD; i += 64 * NW) {
+    const uint32_t c = i / kD, tok = tok0 + c / G, col = (g * G + c % G) * kHd + dbase + i % kD;
+    const float v = lds[i];
+    ((RLH_GLOBAL float*)a.out)[(size_t)tok * qd + col] = v;
+    q8_quant_block32(v, a.out_tiles, tok, col / 32);
   }
+}
+
+template <int NW>
+void launch_pv_pre(hipStream_t st, const AttnArgs& a) {
+  const uint32_t TT = kPvComb / (uint32_t)(a.H / a.KVH);
+  hipLaunchKernelGGL(k_attn_pv_pre<NW>, dim3(a.KVH, (a.n_tok + TT - 1) / TT, 8 / NW), dim3(64 * NW), 0, st, a);
 }
 
 size_t softmax_lds(uint32_t t_max) { return (size_t)((t_max + 3) & ~3u) * 4; }
@@ -1420,8 +1434,14 @@ void launch_attn_pv(hipStream_t st, const AttnArgs& a, bool decode) {
   if (decode) {
     hipLaunchKernelGGL(k_attn_pv_dec, dim3(a.KVH, 4), dim3(512), 0, st, a);
   } else {
-    const uint32_t TT = (uint32_t)(kPreComb / (a.H / a.KVH));
-    hipLaunchKernelGGL(k_attn_pv_pre, dim3(a.KVH, (a.n_tok + TT - 1) / TT), dim3(512), 0, st, a);
+    // eight waves share the probabilities' copies; with fewer than four such
+    // blocks per CU two blocks of half the d each balance better (323 / 332
+    // us at 2048 blocks, 33 / 30 at 128, 7.0 / 6.1 at 192)
+    const uint32_t TT = kPvComb / (uint32_t)(a.H / a.KVH);
+    if ((uint32_t)a.KVH * ((a.n_tok + TT - 1) / TT) >= 1024)
+      launch_pv_pre<8>(st, a);
+    else
+      launch_pv_pre<4>(st, a);
   }
 }
 
