@@ -36,7 +36,6 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <cstdlib>
 #include <type_traits>
 
 #include "attention.h"

@@ -425,18 +425,21 @@ __global__ void __launch_bounds__(256, 4) k_gemm(GemmArgs a0) {
   // read its last row, token tiles past the activation its last tile;
   // neither reaches a kept output. Sources are a uniform base plus 32-bit
   // lane offsets (32 rows' tiles at most apart).
-  const uint32_t rt_bytes = w.ntj * 64 * w.ib, rt0 = r0 / w.tr;
+  // (tile shapes are powers of two: tr = 64 / tj; a division by a value the
+  // compiler does not know costs some forty instructions)
+  const uint32_t tjb = (uint32_t)__builtin_ctz(w.tj), trb = 6 - tjb, trm = w.tr - 1;
+  const uint32_t rt_bytes = w.ntj * 64 * w.ib, rt0 = r0 >> trb;
   const uint8_t* wbase = w.a + (size_t)rt0 * rt_bytes;
   const uint32_t lrow = min(r0 + v.lane % G::kRows, w.rows - 1);  // the lane's row (MT 16: rows 0..31 twice)
-  const uint32_t wlane = (lrow / w.tr - rt0) * rt_bytes + (lrow % w.tr) * 16;
-  const uint32_t tlane = (lrow / w.tr - rt0) * rt_bytes + (((lrow % w.tr) * 2) & ~3u);  // (tr is even)
+  const uint32_t wlane = ((lrow >> trb) - rt0) * rt_bytes + (lrow & trm) * 16;
+  const uint32_t tlane = ((lrow >> trb) - rt0) * rt_bytes + (((lrow & trm) * 2) & ~3u);  // (tr is even)
   const uint32_t last_tile = (a0.n - 1) / 32;
   const uint8_t* xbase[2];
 #pragma unroll
   for (uint32_t t = 0; t < G::kActTiles; t++)
     xbase[t] = a0.x.p + (size_t)min(t0 / 32 + t, last_tile) * nsb * kQ8TileBytes;
   auto copy = [&](uint32_t i, lbyte* buf) {
-    const uint32_t j = i >> 1, h = i & 1, jt = j / w.tj, jr = (j % w.tj) * w.tr;
+    const uint32_t j = i >> 1, h = i & 1, jt = j >> tjb, jr = (j & (w.tj - 1)) << trb;
     const uint8_t* wt = wbase + (size_t)jt * 64 * w.ib + jr * 16;
     const uint32_t xo = j * kQ8TileBytes;
 #pragma unroll
