@@ -1043,11 +1043,11 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
       return gemm_pair_supported(w, w2) || gemm_f32_pair_supported(w, w2);
     };
     auto pair_on = [&](hipStream_t s, const DevMat& w, const DevMat& w2, const Q8Tiles& q8, const float* xf, float* y,
-                       float* y2) {
+                       float* y2, const DevMat* w3 = nullptr, float* y3 = nullptr) {
       if (gemm_supported(w.ty))
-        launch_gemm_pair(s, w, w2, q8, mtok, y, y2);
+        launch_gemm_pair(s, w, w2, q8, mtok, y, y2, w3, y3);
       else
-        launch_gemm_f32_pair(s, w, w2, xf, mtok, n4, y, y2);
+        launch_gemm_f32_pair(s, w, w2, xf, mtok, n4, y, y2, w3, y3);
     };
     auto product = [&](const DevMat& w, const Q8Tiles& q8, const float* xf, float* y, float* resid) {
       product_on(st, w, q8, xf, y, resid);
@@ -1074,7 +1074,12 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
           product_on(s, L.k.dm, c->act_eb, xn, c->kb, nullptr);
         }
       };
-      if (c->side_ok) {
+      if (qk_pair && pair_supported(L.q.dm, L.v.dm)) {
+        // q, k and v of one type (the mixes with one block type): one launch,
+        // no side stream and none of its four event calls, which a short
+        // prompt on a small model spends more time on than on the product
+        pair_on(st, L.q.dm, L.k.dm, c->act_eb, xn, c->qb, c->kb, &L.v.dm, vdst);
+      } else if (c->side_ok) {
         // v (and k, when q and k cannot share a launch) beside q: the side
         // streams start after the norm; the main stream waits for k before
         // the next kernel reads it, and for v there too when v goes

@@ -409,6 +409,11 @@ __global__ void __launch_bounds__(256, 4) k_gemm(GemmArgs a0) {
     resid = nullptr;
     rt = rtg - a0.n_rt1;
   }
+  if (rtg >= a0.n_rt2) {
+    w = a0.w3;
+    y = a0.y3;
+    rt = rtg - a0.n_rt2;
+  }
   const uint32_t t0 = tt * G::kTok, r0 = rt * G::kRows, nsb = w.cols >> 8;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   V v;
@@ -576,16 +581,17 @@ constexpr uint32_t kFT = 16;  // tokens per grouped job
 
 struct GemmF32Args {
   DevMat w;
-  DevMat w2;       // a second segment of the same type and columns (rows 0: none)
+  DevMat w2, w3;   // further segments of the same type and columns (rows 0: none)
   const float* x;  // [n][cols] f32
   uint32_t n;
   float* y;
-  float* y2;
+  float *y2, *y3;
   float* resid;    // of the first segment
   uint32_t n4;     // tokens handled in groups of 4 (n - n % 4)
   uint32_t n_jb;   // blocks per row tile: jobs / 4, rounded up
-  uint32_t n_rt;   // row tiles of both segments
+  uint32_t n_rt;   // row tiles of all segments
   uint32_t n_rt1;  // row tiles of w
+  uint32_t n_rt2;  // row tiles of w and w2
 };
 
 __device__ __forceinline__ float tree8(const float* A) {
@@ -705,6 +711,11 @@ __global__ void __launch_bounds__(256, 3) k_gemm_f32(GemmF32Args a) {
     y = a.y2;
     resid = nullptr;
     r0 = (rtg - a.n_rt1) * kFR;
+  }
+  if (rtg >= a.n_rt2) {
+    w = a.w3;
+    y = a.y3;
+    r0 = (rtg - a.n_rt2) * kFR;
   }
   const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t l = tid & 15, q = (tid >> 4) & 3;
@@ -843,10 +854,11 @@ static void launch_f32_type(hipStream_t st, GemmF32Args a) {
   // 32-row blocks unless they are too few to give every CU two: 2560 x 4096
   // Q5_K with 131 tokens (240 blocks of 32 rows) 52 / 56 us with 16 / 32
   // rows, 19456 x 2560 with 20 (1216) 67 / 61
-  const uint64_t blocks32 = (uint64_t)a.n_jb * ((a.w.rows + 31) / 32 + (a.w2.rows + 31) / 32);
+  const uint64_t blocks32 = (uint64_t)a.n_jb * ((a.w.rows + 31) / 32 + (a.w2.rows + 31) / 32 + (a.w3.rows + 31) / 32);
   const uint32_t fr = blocks32 < 512 ? 16 : 32;
   a.n_rt1 = (a.w.rows + fr - 1) / fr;
-  a.n_rt = a.n_rt1 + (a.w2.rows + fr - 1) / fr;
+  a.n_rt2 = a.n_rt1 + (a.w2.rows + fr - 1) / fr;
+  a.n_rt = a.n_rt2 + (a.w3.rows + fr - 1) / fr;
   const dim3 grid(a.n_jb * ((a.n_rt + 7) / 8) * 8);
   if (fr == 16)
     hipLaunchKernelGGL((k_gemm_f32<TY, 1>), grid, dim3(256), 0, st, a);
@@ -885,8 +897,10 @@ bool gemm_f32_pair_supported(const DevMat& w, const DevMat& w2) {
 }
 
 void launch_gemm_f32_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const float* x, uint32_t n, uint32_t n4,
-                          float* y, float* y2) {
+                          float* y, float* y2, const DevMat* w3, float* y3) {
   GemmF32Args a{};
+  if (w3) a.w3 = *w3;
+  a.y3 = y3;
   a.w = w;
   a.w2 = w2;
   a.x = x;
@@ -914,7 +928,8 @@ static void launch_variant(hipStream_t st, GemmArgs a) {
   using G = Geo<TY, MT>;
   a.n_tt = (a.n + G::kTok - 1) / G::kTok;
   a.n_rt1 = (a.w.rows + G::kRows - 1) / G::kRows;
-  a.n_rt = a.n_rt1 + (a.w2.rows ? (a.w2.rows + G::kRows - 1) / G::kRows : 0);
+  a.n_rt2 = a.n_rt1 + (a.w2.rows + G::kRows - 1) / G::kRows;
+  a.n_rt = a.n_rt2 + (a.w3.rows + G::kRows - 1) / G::kRows;
   const uint32_t blocks = a.n_tt * ((a.n_rt + 7) / 8) * 8;
   hipLaunchKernelGGL((k_gemm<TY, MT>), dim3(blocks), dim3(256), G::kLds, st, a);
 }
@@ -929,7 +944,8 @@ constexpr uint64_t kTiles32 = 1024;
 
 template <uint32_t TY>
 static void launch_type(hipStream_t st, const GemmArgs& a) {
-  const uint64_t tiles = (uint64_t)((a.n + 31) / 32) * ((a.w.rows + 31) / 32 + (a.w2.rows + 31) / 32);
+  const uint64_t tiles =
+      (uint64_t)((a.n + 31) / 32) * ((a.w.rows + 31) / 32 + (a.w2.rows + 31) / 32 + (a.w3.rows + 31) / 32);
   if (tiles < kTiles32)
     launch_variant<TY, 16>(st, a);
   else
@@ -951,8 +967,10 @@ bool gemm_pair_supported(const DevMat& w, const DevMat& w2) {
 }
 
 void launch_gemm_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const Q8Tiles& x, uint32_t n, float* y,
-                      float* y2) {
+                      float* y2, const DevMat* w3, float* y3) {
   GemmArgs a{};
+  if (w3) a.w3 = *w3;
+  a.y3 = y3;
   a.w = w;
   a.w2 = w2;
   a.x = x;
