@@ -28,10 +28,10 @@
 // k_attn_pv_dec (decode): one block per (KV head, 32-wide slice of the head
 // dimension). V slices and probabilities stream through double-buffered LDS
 // chunks while one lane per (head, dimension) runs its ordered saxpy chain.
-// k_attn_pv_pre (prefill): one block per (KV head, tile of query tokens);
-// each V chunk staged in LDS serves every token and head of the tile, and
-// each thread runs eight independent chains. The 32 outputs of a half wave
-// are one Q8 block of the attn_output input in both variants.
+// k_attn_pv_pre (prefill): one block per (KV head, tile of query tokens); the
+// products of a V chunk come from the f32 MFMA, the ordered adds run on the
+// VALU. The 32 outputs of a half wave are one Q8 block of the attn_output
+// input in both variants.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
