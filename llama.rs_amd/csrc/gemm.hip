@@ -298,32 +298,60 @@ struct Step<RLH_TYPE_Q6_K, MT> {
 #pragma unroll
     for (int c = 0; c < 4; c++) b[c] = ((uint64_t)o[c][1] << 32) | o[c][0];
   }
-  __device__ __forceinline__ static void run(const W& v, uint32_t h, float (&acc)[N]) {
-    // the row's f16 in its 4-byte word (even rows low, odd rows high); the
-    // weights enter as 4 q
+  // scale of the row, for weights that enter as 4 q (its f16 sits in a 4-byte
+  // word: even rows low, odd rows high)
+  __device__ __forceinline__ static float scale(const W& v) {
     const uint32_t r = v.row();
-    const float dq = 0.25f * kUnit *
-                     f16_to_f32((*(const RLH_LDS uint32_t*)(v.tail + 4 * r) >> (16 * (r & 1))) & 0xffff);
+    return 0.25f * kUnit * f16_to_f32((*(const RLH_LDS uint32_t*)(v.tail + 4 * r) >> (16 * (r & 1))) & 0xffff);
+  }
+  // terms come in the order s = 0 (c = 0..3), then s = 1 (simd.rs:630-665);
+  // scales[s + 2c] (simd.rs:626-629)
+  //
+  // MT 16, with a wave or two per SIMD and little else to hide an LDS read or
+  // an MFMA behind: the operands of both halves of a super-block are read
+  // first (Half), then four products are issued together and combined (4096
+  // x 12288, 61 tokens: 81 -> 77 us; 2560 x 9728, 237 tokens: 132 -> 123.
+  // The other types have half the products per value and gained nothing).
+  struct Half {
+    float dq, da[4][N];
+    uint64_t sw, a[4], w[4];
+    __device__ __forceinline__ void read(const W& v, uint32_t h) {
+      dq = scale(v);
+      sw = l8(v.chunk(6) + 8 * h);
+#pragma unroll
+      for (int c = 0; c < 4; c++) a[c] = (uint64_t)W::lo64(v.afrag(c));
+      weights(v, 0, w);
+#pragma unroll
+      for (int c = 0; c < 4; c++) v.scales(da[c], c);
+    }
+    __device__ __forceinline__ void combine(const W& v, float (&acc)[N]) const {
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const bool keep = (v.q >> 1) == (uint32_t)s;
+        v4i ci[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) ci[c] = W::dot16(a[c], keep ? w[c] : 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const float ds = dq * (float)(int8_t)(sw >> (8 * (s + 2 * c)));
+#pragma unroll
+          for (int e = 0; e < N; e++) acc[e] = acc[e] + ds * W::dotf(ci[c][e]) * da[c][e];  // simd.rs:663
+        }
+      }
+    }
+  };
+  __device__ __forceinline__ static void run(const W& v, uint32_t h, float (&acc)[N]) {
+    const float dq = scale(v);
     const uint64_t sw = l8(v.chunk(6) + 8 * h);  // the half's 8 scales
-    uint64_t all[4];
-    if constexpr (MT == 16) weights(v, 0, all);
-    // terms in the order s = 0 (c = 0..3), then s = 1 (simd.rs:630-665)
 #pragma unroll
     for (int s = 0; s < 2; s++) {
       uint64_t b[4];
-      if constexpr (MT == 32) {
-        weights(v, s, b);
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; c++) b[c] = (v.q >> 1) == (uint32_t)s ? all[c] : 0;
-      }
+      weights(v, s, b);
       uint64_t a[2];  // the operand and scales of block c + 1 are read while block c is combined
       float da[2][N];
       auto read = [&](int c) {
-        if constexpr (MT == 32)
-          a[c & 1] = l8(v.qs + c * 1024 + v.lane * 16 + 8 * s);
-        else
-          a[c & 1] = (uint64_t)W::lo64(v.afrag(c));
+        a[c & 1] = l8(v.qs + c * 1024 + v.lane * 16 + 8 * s);
         v.scales(da[c & 1], c);
       };
       read(0);
@@ -331,7 +359,7 @@ struct Step<RLH_TYPE_Q6_K, MT> {
       for (int c = 0; c < 4; c++) {
         if (c < 3) read(c + 1);
         const auto ci = W::dot16(a[c & 1], b[c]);
-        const float ds = dq * (float)(int8_t)(sw >> (8 * (s + 2 * c)));  // scales[s + 2c] (simd.rs:626-629)
+        const float ds = dq * (float)(int8_t)(sw >> (8 * (s + 2 * c)));
         float f[N];  // acc + (ds * dot) * da (simd.rs:663)
         phases<N>([&](int e) { f[e] = W::dotf(ci[e]); }, [&](int e) { f[e] = ds * f[e]; },
                   [&](int e) { f[e] = f[e] * da[c & 1][e]; }, [&](int e) { acc[e] = acc[e] + f[e]; });
@@ -510,10 +538,23 @@ __global__ void __launch_bounds__(256, 4) k_gemm(GemmArgs a0) {
       wait_vmcnt<0>();
     lds_barrier();
     if (i + G::kStages - 1 < steps) stage(i + G::kStages - 1, nxt);
-    if (live) {
+    const lbyte* buf = lds + cur * G::kStageBytes;
+    if constexpr (MT == 16 && TY == RLH_TYPE_Q6_K) {
+      if (live) {
+        typename Step<TY, MT>::Half half[2];
+#pragma unroll
+        for (uint32_t h = 0; h < 2; h++) {
+          v.view(buf + h * G::kHalfBytes);
+          half[h].read(v, h);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        half[0].combine(v, acc);
+        half[1].combine(v, acc);
+      }
+    } else if (live) {
 #pragma unroll
       for (uint32_t h = 0; h < G::kHalves; h++) {
-        v.view(lds + cur * G::kStageBytes + h * G::kHalfBytes);
+        v.view(buf + h * G::kHalfBytes);
         Step<TY, MT>::run(v, G::kHalves == 1 ? i & 1 : h, acc);
       }
     }
@@ -937,7 +978,7 @@ static void launch_variant(hipStream_t st, GemmArgs a) {
 // 32 x 32 tiles one per wave fill the SIMDs once from 1024 tiles on; below,
 // 16 x 16 tiles make four times the waves with a quarter of the work each.
 // Both sides measured, 16 / 32: 5120 x 4096 Q4_K, 61 tokens (320 tiles) 23 /
-// 46 us; 2560 x 9728 Q6_K, 237 tokens (640) 134 / 156; 2560 x 4096 Q4_K, 237
+// 46 us; 2560 x 9728 Q6_K, 237 tokens (640) 123 / 155; 2560 x 4096 Q4_K, 237
 // tokens (640) 41 / 47; 5120 x 2560 Q4_K, 237 tokens (1280) 41 / 35; 24576 x
 // 4096 Q4_K, 61 tokens (1536) 68 / 55.
 constexpr uint64_t kTiles32 = 1024;
