@@ -104,7 +104,8 @@ uint64_t rlh_row_bytes(uint32_t ggml_type, uint64_t cols);
 /* Whether this path runs a model of this config, without a device: RLH_OK,
  * RLH_EINVAL (zero dimensions, n_head not a multiple of n_head_kv) or
  * RLH_EUNSUP with the reason (head_dim other than 128, n_embd or n_ff not a
- * multiple of 256, more than 8 query heads per KV head). The reference's
+ * multiple of 256, more than 8 query heads per KV head, an odd n_head: the
+ * rows of attn_output hold a multiple of 256 values). The reference's
  * read_config (src/model.rs:241-293) accepts these shapes; rlh_model_create
  * and rlh_model_load_gguf apply this check before anything is uploaded. */
 int rlh_config_check(const rlh_config* cfg);

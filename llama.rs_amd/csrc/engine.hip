@@ -595,6 +595,12 @@ int rlh_config_check(const rlh_config* cfg) {
                                 "must be multiples of 256");
   if (cfg->n_head / cfg->n_head_kv > (uint32_t)kAttnMaxGroup)
     return fail(RLH_EUNSUP, "more than 8 query heads per KV head");
+  // attn_output's rows: float types are stored as given, so no layout refuses
+  // them, but the products and the Q8 tiles cover whole 256-value items only
+  if ((uint64_t)cfg->n_head * cfg->head_dim % 256 != 0)
+    return fail(RLH_EUNSUP, "n_head " + std::to_string(cfg->n_head) +
+                                ": the rows of attn_output (n_head * head_dim values) must hold a multiple of 256 "
+                                "values, so n_head must be even");
   return RLH_OK;
 }
 
@@ -829,6 +835,8 @@ static int alloc_q8(Q8Buf& b, uint64_t n) {
 }
 
 static int alloc_q8_tiles(Q8Tiles& b, uint64_t n, uint64_t cols) {
+  // the kernels that fill tiles write every 32-value block of a row
+  if (cols % 256 != 0) return fail(RLH_EUNSUP, "Q8 tiles hold rows of a multiple of 256 values");
   if (hipMalloc((void**)&b.p, q8_tiles_bytes(n, cols)) != hipSuccess) return fail(RLH_ENOMEM, "hipMalloc Q8 tiles");
   b.nsb = (uint32_t)(cols / 256);
   return RLH_OK;

@@ -281,6 +281,31 @@ def test_unsupported_shapes_refused_before_upload(tmp_path, shape, reason):
         assert lib.rlh_model_create(ctypes.byref(c), ctypes.byref(hm)) == rlh.RLH_EUNSUP and not hm.value
 
 
+@pytest.mark.parametrize("n_head,n_head_kv", [(1, 1), (3, 1), (3, 3), (5, 5), (7, 1), (21, 3), (63, 9)])
+def test_odd_head_counts_refused_before_upload(tmp_path, n_head, n_head_kv):
+    """attn_output's rows hold n_head * 128 values. Products and Q8 tiles cover
+    whole 256-value items, and a float attn_output has no layout that would
+    refuse a half item, so the config check does: without it a prefill writes
+    the last 128 values of a token's row past its Q8 tiles. Twice the heads
+    pass."""
+    meta = _qwen2_meta(1024, 2048, n_head, n_head_kv, 128)
+    p = tmp_path / "odd.gguf"
+    rlh.write_gguf(p, meta, [("token_embd.weight", rlh.F32, [4, 3], np.zeros(12, np.float32))])
+    lib = rlh.load()
+    with rlh.Gguf(p) as g:
+        c, _ = g.config()
+        assert (c.n_head, c.n_head_kv, c.head_dim) == (n_head, n_head_kv, 128)
+        assert lib.rlh_config_check(ctypes.byref(c)) == rlh.RLH_EUNSUP
+        assert b"attn_output" in lib.rlh_last_error() and b"n_head %d" % n_head in lib.rlh_last_error()
+        h = ctypes.c_void_p()
+        assert lib.rlh_model_load_gguf(g.h, ctypes.byref(h)) == rlh.RLH_EUNSUP
+        assert b"attn_output" in lib.rlh_last_error() and not h.value
+        hm = ctypes.c_void_p()
+        assert lib.rlh_model_create(ctypes.byref(c), ctypes.byref(hm)) == rlh.RLH_EUNSUP and not hm.value
+        c.n_head, c.n_head_kv = 2 * n_head, 2 * n_head_kv
+        assert lib.rlh_config_check(ctypes.byref(c)) == rlh.RLH_OK
+
+
 def test_supported_shapes_pass_config_check():
     """Every benchmark model and every test spec passes rlh_config_check, and
     the checks on zero dimensions and head divisibility come first."""
