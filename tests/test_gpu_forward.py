@@ -320,36 +320,88 @@ def test_prefill_softmax_row_kernels():
     oc.close()
 
 
-@pytest.mark.parametrize("grid_only", ["0", "1"])
-def test_prefill_scores_kernels(monkeypatch, grid_only):
-    """Prefill scores through the persistent kernel (few blocks per CU: every
-    shape here) and, with RLH_QK_PRE_GRID=1, through the kernel with a block
-    per work item: a 4300-token prompt (9 chunks of up to 512 tokens, 4
-    query heads per KV head) and a 600-token prompt continued by 30 tokens
-    at start_pos 600 on small-q4km, logits and the last layer's K/V rows
-    bit-exact against the oracle."""
-    monkeypatch.setenv("RLH_QK_PRE_GRID", grid_only)
-    spec, tensors, m, om = _get("tiny-g4-q4km")
-    prompt = rlh.synth_tokens(91, 4300, spec.vocab)
-    c = m.new_cache(4400)
-    oc = om.new_cache(4400)
-    lg = c.forward_into(prompt, 0)
-    rg = oc.forward_into(prompt, 0, oracle.MODE_BATCH_INT)
-    assert np.array_equal(bits(lg), bits(rg)), f"logits differ (rel {rel_l2(lg, rg):.2e})"
-    c.close()
-    oc.close()
-    spec, tensors, m, om = _get("small-q4km")
-    prompt = rlh.synth_tokens(92, 600, spec.vocab)
-    more = rlh.synth_tokens(93, 30, spec.vocab)
-    c = m.new_cache(700)
-    oc = om.new_cache(700)
-    assert np.array_equal(bits(c.forward_into(prompt, 0)), bits(oc.forward_into(prompt, 0, oracle.MODE_BATCH_INT)))
-    assert np.array_equal(bits(c.forward_into(more, 600)), bits(oc.forward_into(more, 600, oracle.MODE_BATCH_INT)))
-    l = spec.n_layer - 1
-    for which in (0, 1):
-        assert np.array_equal(bits(c.read_kv(l, which, 630)), bits(oc.read_kv(l, which, 630)))
-    c.close()
-    oc.close()
+def _chunks(start, n):
+    return [(start + c, min(512, n - c)) for c in range(0, n, 512)]
+
+
+def _score_tiles(spec, pos, n):
+    """Position tiles per block of the prefill scores kernel for a chunk of n
+    tokens at pos: the most of 8, 4, 2, 1 that leave 512 blocks with work."""
+    per = 64 // (spec.n_head // spec.n_head_kv)
+    for tiles in (8, 4, 2):
+        blocks = sum((pos + min(n, y + per) - 1) // 32 // tiles + 1 for y in range(0, n, per))
+        if blocks * spec.n_head_kv >= 512:
+            return tiles
+    return 1
+
+
+def _pv_waves(spec, n):
+    """Waves per block of the prefill PV kernel."""
+    per = 16 // (spec.n_head // spec.n_head_kv)
+    return 8 if spec.n_head_kv * -(-n // per) >= 1024 else 4
+
+
+def _close_all(*objs):
+    for o in objs:
+        o.close()
+
+
+def _same(got, ref):
+    nan = np.isnan(ref)
+    return np.array_equal(np.isnan(got), nan) and np.array_equal(bits(got[~nan]), bits(ref[~nan]))
+
+
+def _check_prefill(spec, tensors, tokens, parts):
+    """Prefills the parts one after the other on the device and on the oracle:
+    logits after each and every layer's K/V rows bit for bit, NaN exactly
+    where the oracle has NaN. Returns the oracle's K/V rows [layer][k, v] and
+    its last logits."""
+    m, om = rlh.Model(spec, tensors), oracle.OracleModel(spec, tensors)
+    c, oc = m.new_cache(len(tokens) + 8), om.new_cache(len(tokens) + 8)
+    try:
+        at = 0
+        for n in parts:
+            lg = c.forward_into(tokens[at:at + n], at)
+            with np.errstate(all="ignore"):
+                rg = oc.forward_into(tokens[at:at + n], at, oracle.MODE_BATCH_INT)
+            assert _same(lg, rg), f"logits after {at} + {n} tokens differ"
+            at += n
+        rows = []
+        for l in range(spec.n_layer):
+            rows.append([oc.read_kv(l, which, at) for which in (0, 1)])
+            for which in (0, 1):
+                assert _same(c.read_kv(l, which, at), rows[l][which]), f"layer {l} {'kv'[which]} rows differ"
+        return rows, rg
+    finally:
+        _close_all(c, oc, m, om)
+
+
+# Qwen3-14B's 40 / 8 heads: 5 per KV head leave one of 16 combinations of a
+# block empty, and the last block of 509 or 1021 tokens most of them
+_G5_WIDE = rlh.ModelSpec("g5-wide", 2, 256, 512, 40, 8, 1000, True, rlh._q4km(True, rlh.Q4_K, None), n_ctx=4096)
+
+
+@pytest.mark.parametrize("spec,parts,tiles,waves", [
+    (rlh.SPECS["tiny-g4-q4km"], [4300], {1, 2, 4, 8}, {4}),
+    (rlh.SPECS["small-q4km"], [600, 30], {1, 2}, {4}),
+    (_G5_WIDE, [509, 70], {1, 8}, {4, 8}),
+    (_G5_WIDE, [1021], {8}, {8}),
+], ids=["g4-4300", "small-600-30", "g5-509-70", "g5-1021"])
+def test_prefill_scores_kernels(spec, parts, tiles, waves):
+    """The prefill scores kernel with every number of position tiles per block
+    and the PV kernel with both widths, as the chunk lengths and contexts
+    select them (restated above): a 4300-token prompt (9 chunks of up to 512
+    tokens, 4 query heads per KV head), a prompt continued at an odd
+    position, and blocks whose combinations are partly empty. Logits and all
+    K/V rows bit-exact against the oracle."""
+    chunks, at = [], 0
+    for n in parts:
+        chunks += _chunks(at, n)
+        at += n
+    assert {_score_tiles(spec, *c) for c in chunks} == tiles
+    assert {_pv_waves(spec, n) for _, n in chunks} == waves
+    print(f"prefill scores {spec.name} {parts}", flush=True)
+    _check_prefill(spec, rlh.synth_model(spec, 1234), rlh.synth_tokens(91, sum(parts), spec.vocab), parts)
 
 
 def test_nan_logits_argmax_semantics():
