@@ -532,3 +532,70 @@ def test_softmax_walk_replays_bit_exact(n_prompt, monkeypatch):
                     f"mode {mode} step {i}: logits differ (rel {rel_l2(lg, refs[i]):.2e})"
         finally:
             c.close()
+
+
+def _add_biases(spec, tensors, seed):
+    qd, kvd = spec.n_head * spec.head_dim, spec.n_head_kv * spec.head_dim
+    lib = rlh.load()
+    for layer in range(spec.n_layer):
+        for kind, n in ((rlh.T_ATTN_Q_BIAS, qd), (rlh.T_ATTN_K_BIAS, kvd), (rlh.T_ATTN_V_BIAS, kvd)):
+            v = np.empty(n, np.float32)
+            lib.rlh_synth_normal(seed, rlh.tensor_id(kind, layer), 0, n, 0.0, 0.5, v.ctypes.data)
+            tensors.append((kind, layer, rlh.F32, n, 1, v.view(np.uint8)))
+
+
+@pytest.mark.parametrize("ty,biases", [(rlh.Q4_K, False), (rlh.Q6_K, True), (rlh.Q8_0, False), (rlh.Q8_0, True),
+                                       (rlh.Q4_0, True), (rlh.Q5_K, True), (rlh.F16, False), (rlh.F32, True)])
+def test_prefill_one_type_wide(ty, biases):
+    """q, k and v of one type in one launch, and gate and up in one, at sizes
+    that take the large tiles: 499 tokens x 2560 rows are 1280 tiles of 32 x
+    32 (16 x 16 ones below 1024), for the f32 types 8 x 80 blocks of 32 rows
+    (16-row ones below 512). With a v bias the third segment goes to a
+    buffer, without one straight into the cache's rows."""
+    print(f"prefill one type {ty} biases={biases}", flush=True)
+    spec = rlh.ModelSpec("one-type-wide", 2, 512, 1024, 12, 4, 300, True, rlh._all(ty), n_ctx=1024)
+    tensors = rlh.synth_model(spec, 71 + ty)
+    if biases:
+        _add_biases(spec, tensors, 72)
+    _check_prefill(spec, tensors, rlh.synth_tokens(73, 530, spec.vocab), [499, 31])
+
+
+@pytest.mark.parametrize("kind", ["subnormal", "nan", "overflow"])
+def test_prefill_attention_special_values(kind):
+    """K, V, scores and probabilities outside the normal range through the
+    attention products, over rows of several 32-position chunks.
+    subnormal: every K and V value and every p * V product is subnormal or
+    just above (large q and attn_output values bring scores and outputs back).
+    nan: one token's K and V rows are NaN; the tokens before it, whose blocks
+    and chunks hold those rows too, must not see them.
+    overflow: K so large that some scores are infinite: -inf ones take no
+    weight, rows with a +inf one become NaN."""
+    print(f"attention special values: {kind}", flush=True)
+    types = {**rlh._all(rlh.F16), rlh.T_ATTN_V: rlh.F32, rlh.T_ATTN_OUTPUT: rlh.F32, rlh.T_TOKEN_EMBD: rlh.F32}
+    spec = rlh.ModelSpec("special", 2, 256, 512, 8, 2, 500, True, types, n_ctx=512)
+    tensors = rlh.synth_model(spec, 81)
+    tokens = rlh.synth_tokens(82, 171, spec.vocab)
+    first = {k: buf.view(np.float32) for k, l, ty, _, _, buf in tensors if l == 0 and ty == rlh.F32}
+    if kind == "subnormal":
+        first[rlh.T_ATTN_K_NORM][:] *= np.float32(3e-39)
+        first[rlh.T_ATTN_Q_NORM][:] *= np.float32(3e37)
+        first[rlh.T_ATTN_V][:] *= np.float32(1e-38)
+        first[rlh.T_ATTN_OUTPUT][:] *= np.float32(1e38)
+    elif kind == "nan":
+        bad = int(tokens[101])
+        tokens[tokens == bad] = (bad + 1) % spec.vocab
+        tokens[101] = bad
+        first[rlh.T_TOKEN_EMBD].reshape(spec.vocab, -1)[bad, 7] = np.nan
+    else:
+        first[rlh.T_ATTN_K_NORM][:] = 0  # one value per KV head: a score is two products
+        first[rlh.T_ATTN_K_NORM][5] = 6e37
+    rows, logits = _check_prefill(spec, tensors, tokens, [150, 21])
+    v1 = rows[1][1]
+    if kind == "subnormal":
+        tiny = np.finfo(np.float32).tiny
+        assert (np.abs(rows[0][0]) < tiny).mean() > 0.9 and (np.abs(rows[0][1]) < tiny).mean() > 0.9
+        assert np.isfinite(logits).all() and np.abs(v1).max() > 0
+    elif kind == "nan":
+        assert np.isfinite(v1[:101]).all() and np.isnan(v1[101:]).all()
+    else:
+        assert np.isfinite(rows[0][0]).all() and np.isfinite(v1[0]).all() and np.isnan(v1[-1]).any()
