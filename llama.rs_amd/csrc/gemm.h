@@ -16,7 +16,7 @@ struct GemmArgs {
   float* y;        // y[t * rows + r] = total (nullable)
   float* resid;    // resid[t * rows + r] += total (nullable)
   uint32_t n_tt;   // token tiles of the launched variant
-  uint32_t n_rt;   // its row tiles of both segments
+  uint32_t n_rt;   // its row tiles of all segments
   // optional second and third segments of the same type and columns (the q, k
   // and v products of a layer in one launch): row tiles from n_rt1 on belong
   // to w2 and write y2, those from n_rt2 on to w3 and y3 (no residual)
@@ -37,9 +37,10 @@ void launch_gemm(hipStream_t st, const DevMat& w, const Q8Tiles& x, uint32_t n, 
 bool gemm_pair_supported(const DevMat& w, const DevMat& w2);
 void launch_gemm_pair(hipStream_t st, const DevMat& w, const DevMat& w2, const Q8Tiles& x, uint32_t n, float* y,
                       float* y2, const DevMat* w3 = nullptr, float* y3 = nullptr);
-// Weight types without an integer batch path (Q5_K): matmul_batch's f32
-// route on the f32 activations x[n][cols]; the tokens from n4 on (the last
-// n % 4 of the whole batch) take the single-token dot order.
+// Weight types without an integer batch path (Q5_K, Q4_1, Q5_0, Q5_1, F16,
+// BF16, F32): matmul_batch's f32 route on the f32 activations x[n][cols]; the
+// tokens from n4 on (the last n % 4 of the whole batch; all of them for F32
+// weights) take the single-token dot order.
 bool gemm_f32_supported(uint32_t ty);
 void launch_gemm_f32(hipStream_t st, const DevMat& w, const float* x, uint32_t n, uint32_t n4, float* y,
                      float* resid);

@@ -21,7 +21,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-
 #include "gemm.h"
 #include "rlh_device.h"
 
@@ -457,7 +456,7 @@ __global__ void __launch_bounds__(256, 4) k_gemm(GemmArgs a0) {
   // vector-memory count tells which step has landed. Rows past the matrix
   // read its last row, token tiles past the activation its last tile;
   // neither reaches a kept output. Sources are a uniform base plus 32-bit
-  // lane offsets (32 rows' tiles at most apart).
+  // lane offsets (the block's 2 MT rows apart at most).
   // (tile shapes are powers of two: tr = 64 / tj; a division by a value the
   // compiler does not know costs some forty instructions)
   const uint32_t tjb = (uint32_t)__builtin_ctz(w.tj), trb = 6 - tjb, trm = w.tr - 1;
