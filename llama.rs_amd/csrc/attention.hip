@@ -21,7 +21,7 @@
 // k_attn_softmax: one block per (head, token): the row in LDS, max and exp
 // in parallel, the sequential sum in one lane, probabilities written back
 // over the scores.
-// k_attn_softmax_rows (prefill rows up to 4032 positions): 4, 8 or 16
+// k_attn_softmax_rows (prefill rows up to 4988 positions): 4, 8 or 16
 // consecutive tokens of a head per block, one wave per 1, 2 or 4 rows for the
 // parallel parts and the sequential sums of all rows side by side in the
 // lanes of one wave.
@@ -254,6 +254,8 @@ __global__ void __launch_bounds__(256, 2) k_attn_qk(AttnArgs a) {
 // grid: (KVH * ceil(tiles / T), ceil(n_tok / TP)), TP = 64 / G tokens;
 // block 256.
 constexpr uint32_t kQkComb64 = 64, kQkPos = 32;
+// score stores (vector-memory instructions) of a wave per tile that it sees whole
+constexpr uint32_t kQkStores = kQkPos / 16;
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
 __global__ void __launch_bounds__(256, 4) k_attn_qk_pre(AttnArgs a, uint32_t T) {
@@ -298,13 +300,14 @@ __global__ void __launch_bounds__(256, 4) k_attn_qk_pre(AttnArgs a, uint32_t T) 
 #pragma unroll
   for (uint32_t i = 0; i < 8; i++) slot[i] = l * kHd + 4 * ((8 * q + i) ^ l);
   dma(0);
-  bool stored = false;  // the last tile ended with exactly four stores of this wave
+  bool stored = false;  // the last tile ended with the wave's kQkStores stores
   for (uint32_t t = 0; t < nt; t++) {
     // tile t has landed (its copies were issued before the last tile's
-    // stores, which need not be waited for); past the barrier every wave is
-    // done with the other buffer
+    // stores, which need not be waited for: the count must not exceed the
+    // stores that were issued, fewer than that only waits longer); past the
+    // barrier every wave is done with the other buffer
     if (stored)
-      wait_vmcnt<kQkPos / 16>();
+      wait_vmcnt<kQkStores>();
     else
       wait_vmcnt<0>();
     lds_barrier();
