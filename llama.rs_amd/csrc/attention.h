@@ -60,9 +60,9 @@ size_t attn_dec_v_lds(uint32_t t_max, uint32_t group);
 // LDS of the fused decode kernel for t_max positions and `group` query heads
 // per KV head (0 when the rows do not fit).
 size_t attn_dec_fused_lds(uint32_t t_max, uint32_t group);
-// Ordered V accumulation of the probabilities; writes out and its Q8 blocks.
-// decode = one token (d-sliced blocks), else token tiles sharing V chunks.
-void launch_attn_pv(hipStream_t st, const AttnArgs& a, bool decode);
+// Prefill: ordered V accumulation of the probabilities, token tiles sharing V
+// chunks; writes out and its Q8 tiles.
+void launch_attn_pv(hipStream_t st, const AttnArgs& a);
 // Raises the softmax kernel's dynamic LDS limit to cover max_ctx positions.
 bool attn_init(uint32_t max_ctx);
 

@@ -1362,8 +1362,8 @@ size_t softmax_rows_lds(uint32_t t_max, int rw) { return (size_t)4 * rw * softma
 }  // namespace
 
 void launch_attn_scores(hipStream_t st, const AttnArgs& a, bool fused) {
-  const uint32_t ntiles = (a.t_max + kPosTile - 1) / kPosTile;
   if (fused) {
+    const uint32_t ntiles = (a.t_max + kPosTile - 1) / kPosTile;
     hipLaunchKernelGGL(k_attn_qk, dim3(a.KVH * ntiles, a.n_tok), dim3(256), 0, st, a);
   } else {
     const uint32_t TP = kQkComb64 / (uint32_t)(a.H / a.KVH), p0 = a.t_max - a.n_tok, ntiles = (a.t_max + kQkPos - 1) / kQkPos;
@@ -1432,19 +1432,15 @@ void launch_attn_decode(hipStream_t st, const AttnArgs& a, bool f32_out) {
   }
 }
 
-void launch_attn_pv(hipStream_t st, const AttnArgs& a, bool decode) {
-  if (decode) {
-    hipLaunchKernelGGL(k_attn_pv_dec, dim3(a.KVH, 4), dim3(512), 0, st, a);
-  } else {
-    // eight waves share the probabilities' copies; with fewer than four such
-    // blocks per CU two blocks of half the d each balance better (323 / 332
-    // us at 2048 blocks, 33 / 30 at 128, 7.0 / 6.1 at 192)
-    const uint32_t TT = kPvComb / (uint32_t)(a.H / a.KVH);
-    if ((uint32_t)a.KVH * ((a.n_tok + TT - 1) / TT) >= 1024)
-      launch_pv_pre<8>(st, a);
-    else
-      launch_pv_pre<4>(st, a);
-  }
+void launch_attn_pv(hipStream_t st, const AttnArgs& a) {
+  // eight waves share the probabilities' copies; with fewer than four such
+  // blocks per CU two blocks of half the d each balance better (323 / 332
+  // us at 2048 blocks, 33 / 30 at 128, 7.0 / 6.1 at 192)
+  const uint32_t TT = kPvComb / (uint32_t)(a.H / a.KVH);
+  if ((uint32_t)a.KVH * ((a.n_tok + TT - 1) / TT) >= 1024)
+    launch_pv_pre<8>(st, a);
+  else
+    launch_pv_pre<4>(st, a);
 }
 
 bool attn_init(uint32_t max_ctx) {

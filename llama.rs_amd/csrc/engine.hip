@@ -1139,7 +1139,7 @@ static int forward_batch_impl(rlh_model* m, rlh_cache* c, const uint32_t* tokens
       launch_attn_scores(st, a, false);
       launch_attn_softmax(st, a);
       if (v_pending) HIPCHK(hipStreamWaitEvent(st, c->ev_join[1], 0));
-      launch_attn_pv(st, a, false);
+      launch_attn_pv(st, a);
       product(L.o.dm, c->act_qb, c->attnb, nullptr, c->xb);
       launch_rmsnorm_q8(st, c->xb, L.ffn_norm.p, E, mtok, eps, c->act_eb, xn);
       if (pair_supported(L.gate.dm, L.up.dm)) {  // one launch of both (one boundary less)
