@@ -891,19 +891,41 @@ template <uint32_t TY>
 static void launch_f32_type(hipStream_t st, GemmF32Args a) {
   const uint32_t jobs = (a.n4 + kFT - 1) / kFT + (a.n - a.n4 + 3) / 4;
   a.n_jb = (jobs + 3) / 4;
-  // 32-row blocks unless they are too few to give every CU two: 2560 x 4096
-  // Q5_K with 131 tokens (240 blocks of 32 rows) 52 / 56 us with 16 / 32
-  // rows, 19456 x 2560 with 20 (1216) 67 / 61
-  const uint64_t blocks32 = (uint64_t)a.n_jb * ((a.w.rows + 31) / 32 + (a.w2.rows + 31) / 32 + (a.w3.rows + 31) / 32);
-  const uint32_t fr = blocks32 < 512 ? 16 : 32;
-  a.n_rt1 = (a.w.rows + fr - 1) / fr;
-  a.n_rt2 = a.n_rt1 + (a.w2.rows + fr - 1) / fr;
-  a.n_rt = a.n_rt2 + (a.w3.rows + fr - 1) / fr;
+  auto row_tiles = [&](uint32_t fr) {
+    a.n_rt1 = (a.w.rows + fr - 1) / fr;
+    a.n_rt2 = a.n_rt1 + (a.w2.rows + fr - 1) / fr;
+    a.n_rt = a.n_rt2 + (a.w3.rows + fr - 1) / fr;
+  };
+  // 32-row or 16-row blocks. A block whose every wave multiplies most of the
+  // time (four jobs; three for F32 weights, whose jobs are all 4 single
+  // tokens) takes about 14 / 23 / 33 us of 1024 columns with one / two / three
+  // of 32 rows on a CU and 13 / 20 / 28 / 38 with one to four of 16, so 32
+  // rows unless 16 put no more blocks on a CU (an XCD's 32 CUs get every
+  // eighth row tile). Both sides, 16 / 32 rows: F32 3072 columns, 131 tokens,
+  // 128 blocks of 32 rows 51 / 33, 256 (two on some CUs either way) 51 / 57;
+  // 200 tokens, 416 blocks 108 / 57; Q5_K 4096 columns, 200 tokens, 320 blocks
+  // 94 / 88.
+  // The others overlap up to what is resident. Three jobs, or the types whose
+  // dequantizing takes longest: 16 rows until a second round of the three per
+  // CU begins (Q5_K 3072 columns, 131 tokens, 384 blocks 55 / 65, 400 77 / 65;
+  // Q5_0 4096 columns, 200 tokens, 384 92 / 96, 448 124 / 96). One or two jobs:
+  // a little longer (3072 columns, 20 tokens, 512 blocks Q4_1 44 / 61, Q5_K 64
+  // / 65; 576 F16 61 / 60, Q5_K 76 / 71).
+  const uint32_t per = (jobs + a.n_jb - 1) / a.n_jb;
+  auto on_cu = [&] { return (a.n_jb * (uint64_t)((a.n_rt + 7) / 8) + 31) / 32; };
+  row_tiles(16);
+  const uint64_t on_cu16 = on_cu();
+  row_tiles(32);
+  const uint64_t blocks32 = (uint64_t)a.n_jb * a.n_rt;
+  constexpr bool kSlowDq = TY == RLH_TYPE_Q5_0 || TY == RLH_TYPE_Q5_1;
+  const bool busy = (per == 4 && !kSlowDq) || (per == 3 && TY == RLH_TYPE_F32);
+  const bool rows32 = busy ? on_cu16 > on_cu() : blocks32 > (per >= 3 ? 384 : 511);
+  if (!rows32) row_tiles(16);
   const dim3 grid(a.n_jb * ((a.n_rt + 7) / 8) * 8);
-  if (fr == 16)
-    hipLaunchKernelGGL((k_gemm_f32<TY, 1>), grid, dim3(256), 0, st, a);
-  else
+  if (rows32)
     hipLaunchKernelGGL((k_gemm_f32<TY, 2>), grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_gemm_f32<TY, 1>), grid, dim3(256), 0, st, a);
 }
 
 static void launch_gemm_f32_args(hipStream_t st, GemmF32Args a) {

@@ -550,8 +550,9 @@ def test_prefill_one_type_wide(ty, biases):
     """q, k and v of one type in one launch, and gate and up in one, at sizes
     that take the large tiles: 499 tokens x 2560 rows are 1280 tiles of 32 x
     32 (16 x 16 ones below 1024), for the f32 types 8 x 80 blocks of 32 rows
-    (16-row ones below 512). With a v bias the third segment goes to a
-    buffer, without one straight into the cache's rows."""
+    (the 16-row ones would put five on a CU against three). With a v bias the
+    third segment goes to a buffer, without one straight into the cache's
+    rows."""
     print(f"prefill one type {ty} biases={biases}", flush=True)
     spec = rlh.ModelSpec("one-type-wide", 2, 512, 1024, 12, 4, 300, True, rlh._all(ty), n_ctx=1024)
     tensors = rlh.synth_model(spec, 71 + ty)

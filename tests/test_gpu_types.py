@@ -118,6 +118,23 @@ def test_matmul_batch_job_edges_bit_exact(ty, rows, cols, n):
     assert np.array_equal(bits(got), bits(ref))
 
 
+# Both sides of the choice between 16-row and 32-row blocks (the second of
+# each pair of sizes takes 32): four jobs per block with one or two 16-row
+# blocks per CU, three jobs at the end of the resident 16-row blocks, and F32
+# weights (four single tokens a job) with two or three per CU.
+@pytest.mark.parametrize("ty,rows,n", [(F16, 4096, 64), (F16, 4097, 64), (13, 4097, 61), (13, 12288, 48),
+                                       (13, 12289, 48), (F32, 896, 131), (F32, 897, 131), (F32, 4097, 10)])
+def test_matmul_batch_block_rows_bit_exact(ty, rows, n):
+    cols = 512
+    print(f"ty={ty} matmul_batch {rows}x{cols} n={n}", flush=True)
+    rng = np.random.default_rng(rows + n + ty)
+    w = random_blocks(ty, rows * cols // BLOCK[ty][0], rng)
+    xs = rng.standard_normal((n, cols)).astype(np.float32)
+    got = rlh.matmul_batch(ty, w, rows, cols, xs, n)
+    ref = oracle.matmul_batch(ty, w, rows, cols, xs, n, oracle.MODE_BATCH_INT)
+    assert np.array_equal(bits(got), bits(ref))
+
+
 @pytest.mark.parametrize("ty", TYPES + [13], ids=[NAMES[t] for t in TYPES] + ["Q5_K"])
 def test_matmul_batch_non_finite_activations(ty):
     """Infinite, NaN, subnormal and huge activations through the FMA chains."""
