@@ -1434,8 +1434,10 @@ void launch_attn_decode(hipStream_t st, const AttnArgs& a, bool f32_out) {
 
 void launch_attn_pv(hipStream_t st, const AttnArgs& a) {
   // eight waves share the probabilities' copies; with fewer than four such
-  // blocks per CU two blocks of half the d each balance better (323 / 332
-  // us at 2048 blocks, 33 / 30 at 128, 7.0 / 6.1 at 192)
+  // blocks per CU two blocks of half the d each balance better. us with eight
+  // / four waves, contexts of 1000: 384 blocks 53 / 46, 512 56 / 56, 640 76 /
+  // 67, 768 80 / 81, 1024 107 / 108, 1280 119 / 121, 2048 195 / 199; contexts
+  // of 3584: 1280 357 / 375, 2048 573 / 616.
   const uint32_t TT = kPvComb / (uint32_t)(a.H / a.KVH);
   if ((uint32_t)a.KVH * ((a.n_tok + TT - 1) / TT) >= 1024)
     launch_pv_pre<8>(st, a);

@@ -998,10 +998,12 @@ static void launch_variant(hipStream_t st, GemmArgs a) {
 
 // 32 x 32 tiles one per wave fill the SIMDs once from 1024 tiles on; below,
 // 16 x 16 tiles make four times the waves with a quarter of the work each.
-// Both sides measured, 16 / 32: 5120 x 4096 Q4_K, 61 tokens (320 tiles) 23 /
-// 46 us; 2560 x 9728 Q6_K, 237 tokens (640) 123 / 155; 2560 x 4096 Q4_K, 237
-// tokens (640) 41 / 47; 5120 x 2560 Q4_K, 237 tokens (1280) 41 / 35; 24576 x
-// 4096 Q4_K, 61 tokens (1536) 68 / 55.
+// Both sides measured, 16 / 32, us at 512, 1024, 1152 and 2048 tiles (4096
+// columns, 237 tokens; the ratios are the same within 4 % from 1024 to 12288
+// columns and with 61 and 509 tokens): Q4_K 22 / 45, 42 / 46, 57 / 49, 79 / 51;
+// Q6_K 31 / 64, 61 / 65, 77 / 73, 115 / 75; Q8_0 18 / 36, 35 / 37, 45 / 42, 66
+// / 44; Q4_0 20 / 36, 39 / 37, 52 / 40, 74 / 41 (equal at 768 already, at most
+// 5 % lost in between).
 constexpr uint64_t kTiles32 = 1024;
 
 template <uint32_t TY>
