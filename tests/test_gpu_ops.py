@@ -179,6 +179,20 @@ def test_matmul_batch_tiles_bit_exact(ty, rows, cols, n):
     assert np.array_equal(bits(got), bits(ref))
 
 
+@pytest.mark.parametrize("n", [65504, 65505, 65570])
+def test_matmul_batch_quantizes_long_batches_in_parts(n):
+    """More tokens than one grid of the tiled quantizer holds (65504): the
+    rows from there on go in a launch of their own, at a tile's start."""
+    print(f"matmul_batch long batch n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    rows, cols = 20, 256
+    w = random_blocks(Q8_0, rows * cols // BLOCK[Q8_0][0], rng)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    got = rlh.matmul_batch(Q8_0, w, rows, cols, x, n)
+    ref = oracle.matmul_batch(Q8_0, w, rows, cols, x, n, oracle.MODE_BATCH_INT)
+    assert np.array_equal(bits(got), bits(ref))
+
+
 @pytest.mark.parametrize("ty", TYPES)
 @pytest.mark.parametrize("rows,n", [(40, 37), (2100, 500)])
 def test_matmul_batch_special_scales(ty, rows, n):
